@@ -248,8 +248,11 @@ int srq_had_sign_quant_bf6(const void *x, int64_t rows, int64_t n, int64_t K,
  * uint4 quantizer of srq_asym_quant_dynamic (row min/max of the rotated,
  * signed fp16 values, scale, zero point, codes): q u8 [rows, n/2], scale
  * and zero f16 [rows].  Bit-identical to srq_online_hadamard followed by
- * srq_asym_quant_dynamic.  Needs K % 4 == 0 and n = K * 512 or K * 1024
- * (9 <= K <= 32), else SRQ_EUNSUPPORTED.  Replaces OnlineHadamard followed
+ * srq_asym_quant_dynamic.  Needs an MFMA form of the rotation, else
+ * SRQ_EUNSUPPORTED: K % 4 == 0 and n = K * 512 or K * 1024 with 9 <= K <= 32,
+ * or hadK 8-byte aligned and n = K * 64 or K * 128 <= 20480 with
+ * 12 <= K <= 176, n = K * 256 with 12 <= K <= 64 or n = K * 512 with
+ * 36 <= K <= 64.  Replaces OnlineHadamard followed
  * by AsymQuantizer (signrot/nn/hadamard.py:26-42, nn/quantization.py:59-67,
  * kernels/fused.cu:143-195); the reference has no fused form. */
 int srq_had_sign_asym_quant(const void *x, int64_t rows, int64_t n, int64_t K,

@@ -486,8 +486,15 @@ def had_sign_quant(x, hadK, K, sign=None, clip_ratio=1.0, fp32_had=False):
 
 
 def had_asym_fusable(n, K):
-    """Whether had_sign_asym_quant has a one-launch kernel for n = K x 2^k."""
-    return K % 4 == 0 and 9 <= K <= 32 and n in (K * 512, K * 1024)
+    """Whether had_sign_asym_quant has a one-launch kernel for n = K x 2^k
+    (had_sign_asym_quant also needs hadK 8-byte aligned, as a tensor of its
+    own is)."""
+    if K % 4 == 0 and 9 <= K <= 32 and n in (K * 512, K * 1024):
+        return True
+    if K % 4 or not 12 <= K <= 176:
+        return False
+    return (n in (K * 64, K * 128) and (n <= 20480 or K <= 64)) or \
+        (n == K * 256 and K <= 64) or (n == K * 512 and 32 < K <= 64)
 
 
 def had_sign_asym_quant(x, hadK, K, sign=None, clip_ratio=1.0):
@@ -500,7 +507,7 @@ def had_sign_asym_quant(x, hadK, K, sign=None, clip_ratio=1.0):
     n = x.shape[-1]
     _check_had("had_sign_asym_quant", n, hadK, K, sign, False)
     rows = x.numel() // n if n else 0
-    if not had_asym_fusable(n, K):
+    if not had_asym_fusable(n, K) or hadK.data_ptr() % 8:
         rot = online_hadamard(x.reshape(rows, n), hadK, K, sign)
         q, s, z = asym_quant_dynamic(rot, clip_ratio)
         return (q.view(*x.shape[:-1], -1), s.view(*x.shape[:-1], 1),

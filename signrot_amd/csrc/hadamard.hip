@@ -408,6 +408,10 @@ int srq_had512_mfma(const void *x, int64_t rows, int64_t n, int64_t K, const voi
                     const int32_t *sign_row = nullptr, int64_t n_sign_rows = 0,
                     void *qzero = nullptr, int bf6 = 0);
 
+int srq_had_kron_mfma(const void *x, int64_t rows, int64_t n, int64_t K, const void *hadK,
+                      const int8_t *sign, float clip, void *q, void *qscale, void *qzero,
+                      void *out, hipStream_t st);
+
 // Rotation + sign + quantizer of rows of n = 256 E (a power of two, K = 1:
 // the plain FWHT) for the decode-sized row counts of a q/k/v-shaped
 // QLinear: one 256-thread block per row, thread t holding elements
@@ -595,7 +599,10 @@ extern "C" int srq_online_hadamard(const void *x, void *out, int64_t rows, int64
     a.scale = 1.0f / sqrtf((float)n);
     a.fp32_had = fp32_had ? 1 : 0;
     if (!fp32_had &&
-        srq_had512_mfma(x, rows, n, K, hadK, sign, 1.f, nullptr, nullptr, out, (hipStream_t)stream)) {
+        (srq_had512_mfma(x, rows, n, K, hadK, sign, 1.f, nullptr, nullptr, out,
+                         (hipStream_t)stream) ||
+         srq_had_kron_mfma(x, rows, n, K, hadK, sign, 1.f, nullptr, nullptr, nullptr, out,
+                           (hipStream_t)stream))) {
         SRQ_LAUNCH_CHECK("online_hadamard");
         return SRQ_OK;
     }
@@ -625,8 +632,10 @@ extern "C" int srq_had_sign_quant(const void *x, int64_t rows, int64_t n, int64_
     a.clip = clip_ratio;
     a.q = (uint32_t *)q;
     a.qscale = (f16 *)scale;
-    if (!fp32_had && srq_had512_mfma(x, rows, n, K, hadK, sign, clip_ratio, q, scale, nullptr,
-                                     (hipStream_t)stream)) {
+    if (!fp32_had && (srq_had512_mfma(x, rows, n, K, hadK, sign, clip_ratio, q, scale, nullptr,
+                                      (hipStream_t)stream) ||
+                      srq_had_kron_mfma(x, rows, n, K, hadK, sign, clip_ratio, q, scale, nullptr,
+                                        nullptr, (hipStream_t)stream))) {
         SRQ_LAUNCH_CHECK("had_sign_quant");
         return SRQ_OK;
     }
@@ -743,11 +752,13 @@ extern "C" int srq_had_sign_asym_quant(const void *x, int64_t rows, int64_t n, i
     SRQ_CHECK_ARG(srq_aligned(x, 16) && srq_aligned(q, 16),
                   "had_sign_asym_quant: x and q must be 16-byte aligned");
     if (srq_had512_mfma(x, rows, n, K, hadK, sign, clip_ratio, q, scale, nullptr,
-                        (hipStream_t)stream, nullptr, 0, nullptr, 0, zero)) {
+                        (hipStream_t)stream, nullptr, 0, nullptr, 0, zero) ||
+        srq_had_kron_mfma(x, rows, n, K, hadK, sign, clip_ratio, q, scale, zero, nullptr,
+                          (hipStream_t)stream)) {
         SRQ_LAUNCH_CHECK("had_sign_asym_quant");
         return SRQ_OK;
     }
-    srq_set_error("had_sign_asym_quant: needs K %% 4 == 0 and n = K * 512 or K * 1024 with "
-                  "9 <= K <= 32 (n=%lld, K=%lld)", (long long)n, (long long)K);
+    srq_set_error("had_sign_asym_quant: no fused form for n=%lld, K=%lld", (long long)n,
+                  (long long)K);
     return SRQ_EUNSUPPORTED;
 }
