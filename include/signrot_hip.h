@@ -382,6 +382,21 @@ int srq_qkv_rope_had_append(const void *qkv, const void *cos, const void *sin,
                             const int32_t *last_page_offset, int64_t num_layers,
                             int64_t layer_idx, int64_t page_size, void *stream);
 
+/* The prefill form: qkv f16 [batch, seq_len, (Hq + 2 Hk) * head_dim], the
+ * projection output of a prompt without padding, cos/sin f16 [cos_batch,
+ * seq_len, head_dim].  In place in qkv: RoPE of the q and k rows.  Into the
+ * cache: k (after RoPE and, when `rotate`, the head-dim Hadamard times
+ * had_scale) and v quantized, token t of a request at position
+ * length - seq_len + t of the index tensors.  Bit-identical to srq_rope_qk,
+ * srq_hadamard_transform of k, srq_kv_quant_pack and srq_init_kv_i4 in turn
+ * (modeling_llama.py:62-79, signrot/transformers/kv_cache.py:295-395). */
+int srq_prefill_qkv_cache(void *qkv, const void *cos, const void *sin, int64_t cos_batch,
+                          int64_t batch, int64_t seq_len, int64_t n_q_heads, int64_t n_kv_heads,
+                          int64_t head_dim, float had_scale, int rotate, void *kv_data,
+                          void *kv_param, const int32_t *kv_indptr, const int32_t *kv_indices,
+                          const int32_t *last_page_offset, int64_t num_layers, int64_t layer_idx,
+                          int64_t page_size, void *stream);
+
 /* srq_qkv_rope_had_append followed by srq_batch_decode_i4, in one launch:
  * each decode block (request, KV head, chunk) computes the rotated q rows of
  * its query-head group from qkv and keeps them on chip, and the block whose

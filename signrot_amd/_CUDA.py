@@ -23,6 +23,7 @@ Added ops (no reference counterpart, fused forms of reference chains):
   qkv_rope_had_append   = rope_qk + K/q Hadamard + kv_quant_pack + append_kv_i4
                                                               kv_cache.py:144-170, 295-415
   qkv_decode_i4         = qkv_rope_had_append + batch_decode_i4 kv_cache.py:144-170, 295-415
+  prefill_qkv_cache     = rope_qk + K Hadamard + kv_quant_pack + init_kv_i4 kv_cache.py:295-395
 """
 import functools
 
@@ -617,6 +618,29 @@ def qkv_rope_had_append(qkv, cos, sin, n_q_heads, n_kv_heads, kv_data, kv_param,
           _ptr(kv_param), _ptr(kv_indptr), _ptr(kv_indices), _ptr(last_page_offset), L,
           int(layer_idx), P, _stream(qkv))
     return q
+
+
+def prefill_qkv_cache(qkv, cos, sin, n_q_heads, kv_data, kv_param, kv_indptr, kv_indices,
+                      last_page_offset, layer_idx, had_scale, rotate=True):
+    """Prefill q/k/v post-processing of qkv f16 [B, T, (Hq + 2 Hk) * 128] (no
+    padding), in place: RoPE of the q and k rows; k (after RoPE and, when
+    `rotate`, the head-dim Hadamard times had_scale) and v are quantized into
+    the cache as each request's last T tokens.  cos / sin [1 or B, T, 128]."""
+    L, H, P, D = _check_cache("prefill_qkv_cache", kv_data, kv_param, kv_indptr, kv_indices,
+                              last_page_offset)
+    _check("prefill_qkv_cache", [(qkv, "qkv"), (cos, "cos"), (sin, "sin"), (kv_data, "kv_data")],
+           [torch.float16, torch.float16, torch.float16, None])
+    if qkv.dim() != 3 or qkv.shape[2] != (n_q_heads + 2 * H) * D:
+        raise RuntimeError(f"prefill_qkv_cache: qkv must be [B, T, {(n_q_heads + 2 * H) * D}]")
+    B, T = qkv.shape[:2]
+    if kv_indptr.shape[0] != B + 1 or last_page_offset.shape[0] != B:
+        raise RuntimeError("prefill_qkv_cache: index tensors do not match the batch")
+    if cos.shape != sin.shape or tuple(cos.shape) not in ((1, T, D), (B, T, D)):
+        raise RuntimeError(f"prefill_qkv_cache: cos/sin must be [1 or {B}, {T}, {D}]")
+    _call("srq_prefill_qkv_cache", _ptr(qkv), _ptr(cos), _ptr(sin), cos.shape[0], B, T,
+          int(n_q_heads), H, D, float(had_scale), 1 if rotate else 0, _ptr(kv_data),
+          _ptr(kv_param), _ptr(kv_indptr), _ptr(kv_indices), _ptr(last_page_offset), L,
+          int(layer_idx), P, _stream(qkv))
 
 
 def batch_decode_i4(o, q, kv_data, kv_param, kv_indptr, kv_indices, last_page_offset,

@@ -132,42 +132,47 @@ SRQ_DEV float xor_lane(float v, int m) { return __shfl_xor(v, m, 64); }
 // 16-lane group holds dims 8 l .. 8 l + 7 of one D = 128 row in v; kind 0 / 1
 // / 2 = q / k / v row.  Every lane of the wave must call these (shuffles).
 // RoPE (q, k), then FWHT_D * had_scale rounded to fp16 (q, k, when rotate).
-SRQ_DEV void qkv_row_transform(float (&v)[8], int kind, int l, const f16 *cs, const f16 *sn,
-                               int64_t ct, float had_scale, int rotate) {
+SRQ_DEV void qkv_row_rope(float (&v)[8], int kind, int l, const f16 *cs, const f16 *sn,
+                          int64_t ct) {
     constexpr int D = 128;
-    {
-        float y[8];
+    float y[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float o = xor_lane(v[e], 8);
+        const int i = 8 * l + e;
+        const f16 c = cs[ct * D + i], s = sn[ct * D + i];
+        const f16 xe = (f16)v[e], xo = (f16)o;  // exact: both came from fp16
+        y[e] = (float)(l < 8 ? rope_lo(xe, xo, c, s) : rope_hi(xo, xe, c, s));
+    }
+    if (kind != 2) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = y[e];
+    }
+}
+
+SRQ_DEV void qkv_row_had(float (&v)[8], int kind, int l, float had_scale) {
+    float w[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w[e] = v[e];
+    fwht_regs<8>(w);
+#pragma unroll
+    for (int m = 1; m < 16; m <<= 1) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const float o = xor_lane(v[e], 8);
-            const int i = 8 * l + e;
-            const f16 c = cs[ct * D + i], s = sn[ct * D + i];
-            const f16 xe = (f16)v[e], xo = (f16)o;  // exact: both came from fp16
-            y[e] = (float)(l < 8 ? rope_lo(xe, xo, c, s) : rope_hi(xo, xe, c, s));
-        }
-        if (kind != 2) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = y[e];
+            const float o = xor_lane(w[e], m);
+            w[e] = (l & m) ? o - w[e] : w[e] + o;
         }
     }
-    if (rotate) {
-        float w[8];
+    if (kind != 2) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) w[e] = v[e];
-        fwht_regs<8>(w);
-#pragma unroll
-        for (int m = 1; m < 16; m <<= 1) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float o = xor_lane(w[e], m);
-                w[e] = (l & m) ? o - w[e] : w[e] + o;
-            }
-        }
-        if (kind != 2) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = (float)f16_rn(w[e] * had_scale);
-        }
+        for (int e = 0; e < 8; ++e) v[e] = (float)f16_rn(w[e] * had_scale);
     }
+}
+
+SRQ_DEV void qkv_row_transform(float (&v)[8], int kind, int l, const f16 *cs, const f16 *sn,
+                               int64_t ct, float had_scale, int rotate) {
+    qkv_row_rope(v, kind, l, cs, sn, ct);
+    if (rotate) qkv_row_had(v, kind, l, had_scale);
 }
 
 // KV int4 quantizer of a transformed row: the row max / min over the 16
@@ -237,6 +242,66 @@ __global__ __launch_bounds__(256) void qkv_post_kernel(QkvArgs a, Paged p) {
     const int64_t h = slot - a.hq - (kind == 2 ? a.hk : 0);
     const int64_t entry = pos % p.page;
     const int64_t ri = row_index(p, page, kv, h, entry);
+    reinterpret_cast<u32 *>(p.data + ri * (D / 2))[l] = word;
+    if (l == 0) reinterpret_cast<uint32_t *>(p.param)[ri] = pack_param(scale, zero);
+}
+
+// The prefill form: T tokens per request, between the q/k/v projection and
+// the prefill attention (modeling_llama.py:62-90, kv_cache.py:295-395).  RoPE
+// of the q and k rows in place in the projection output, which the attention
+// then reads strided; k (RoPE'd, head-dim FWHT) and v quantized straight into
+// their cache slots, token t of a request at position len - T + t.  The same
+// arithmetic as rope_qk, hadamard_transform, kv_quant_pack and init_kv_i4 in
+// turn, one pass over the projection output instead of copies of the q, k
+// and v slices and a pass each.  Sixteen lanes per 128-wide row as above; the
+// rotation and the quantizer run only in waves that hold a k or v row.
+// 8B widths (32 + 2 x 8 heads), T = 2048: the ops it stands
+// for took 17 (slices) + 22 (RoPE) + 13 (FWHT) + 2 x 4.8 (quantizers) + 5.7 us
+// (cache fill).
+struct PrefillQkvArgs {
+    f16 *qkv;              // [B, T, hq + 2 hk, D]
+    const f16 *cs, *sn;    // [cos_batch, T, D]
+    int cos_batch;
+    int64_t B, T;
+    int hq, hk;
+    float had_scale;
+    int rotate;
+};
+
+__global__ __launch_bounds__(256) void prefill_qkv_kernel(PrefillQkvArgs a, Paged p) {
+    constexpr int D = 128;
+    const int l = threadIdx.x & 15;
+    const int hs = a.hq + 2 * a.hk;
+    const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+    const bool valid = row < a.B * a.T * hs;
+    const int64_t tok = valid ? row / hs : 0;
+    const int slot = valid ? (int)(row - tok * hs) : 0;
+    const int kind = slot < a.hq ? 0 : (slot < a.hq + a.hk ? 1 : 2);  // q, k, v
+    const int64_t b = tok / a.T, t = tok - b * a.T;
+    v8h x = valid ? *reinterpret_cast<const v8h *>(a.qkv + row * D + 8 * l) : (v8h){};
+    int64_t pos = -1, page = 0;
+    if (valid && kind != 0) {
+        pos = seq_len_of(p, b) - a.T + t;
+        if (pos >= 0) page = p.indices[p.indptr[b] + pos / p.page];
+    }
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (float)x[e];
+    if (__builtin_amdgcn_ballot_w64(kind != 2) != 0) {
+        qkv_row_rope(v, kind, l, a.cs, a.sn, a.cos_batch == 1 ? t : tok);
+        if (valid && kind != 2) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) x[e] = (f16)v[e];
+            *reinterpret_cast<v8h *>(a.qkv + row * D + 8 * l) = x;
+        }
+    }
+    if (__builtin_amdgcn_ballot_w64(kind != 0) == 0) return;  // q rows only
+    if (a.rotate) qkv_row_had(v, kind, l, a.had_scale);
+    f16 scale, zero;
+    const u32 word = kv_row_codes(v, scale, zero);
+    if (!valid || kind == 0 || pos < 0) return;
+    const int64_t h = slot - a.hq - (kind == 2 ? a.hk : 0);
+    const int64_t ri = row_index(p, page, kind - 1, h, pos % p.page);
     reinterpret_cast<u32 *>(p.data + ri * (D / 2))[l] = word;
     if (l == 0) reinterpret_cast<uint32_t *>(p.param)[ri] = pack_param(scale, zero);
 }
@@ -1308,6 +1373,45 @@ extern "C" int srq_qkv_rope_had_append(const void *qkv, const void *cos, const v
     const int64_t blocks = srq_cdiv(rows, 16);
     SRQ_CHECK_ARG(blocks <= 0x7fffffffLL, "%s: too many rows", name);
     qkv_post_kernel<<<dim3((unsigned)blocks), 256, 0, (hipStream_t)stream>>>(a, p);
+    SRQ_LAUNCH_CHECK(name);
+    return SRQ_OK;
+}
+
+extern "C" int srq_prefill_qkv_cache(void *qkv, const void *cos, const void *sin,
+                                     int64_t cos_batch, int64_t batch, int64_t seq_len,
+                                     int64_t n_q_heads, int64_t n_kv_heads, int64_t head_dim,
+                                     float had_scale, int rotate, void *kv_data, void *kv_param,
+                                     const int32_t *kv_indptr, const int32_t *kv_indices,
+                                     const int32_t *last_page_offset, int64_t num_layers,
+                                     int64_t layer_idx, int64_t page_size, void *stream) {
+    const char *name = "prefill_qkv_cache";
+    int rc = check_paged(name, kv_data, kv_param, kv_indptr, kv_indices, last_page_offset,
+                         num_layers, layer_idx, n_kv_heads, page_size, head_dim);
+    if (rc) return rc;
+    SRQ_CHECK_ARG(batch >= 0 && batch <= 65535 && seq_len >= 0 && n_q_heads > 0 &&
+                      n_kv_heads > 0 && n_q_heads <= 1024 && n_kv_heads <= 1024,
+                  "%s: bad batch, length or head counts", name);
+    SRQ_CHECK_ARG(cos_batch == 1 || cos_batch == batch, "%s: cos/sin batch must be 1 or B",
+                  name);
+    if (batch == 0 || seq_len == 0) return SRQ_OK;
+    SRQ_CHECK_ARG(qkv && cos && sin, "%s: null pointer", name);
+    SRQ_CHECK_ARG(srq_aligned(qkv, 16), "%s: qkv must be 16-byte aligned", name);
+    PrefillQkvArgs a;
+    a.qkv = (f16 *)qkv;
+    a.cs = (const f16 *)cos;
+    a.sn = (const f16 *)sin;
+    a.cos_batch = (int)cos_batch;
+    a.B = batch;
+    a.T = seq_len;
+    a.hq = (int)n_q_heads;
+    a.hk = (int)n_kv_heads;
+    a.had_scale = had_scale;
+    a.rotate = rotate ? 1 : 0;
+    Paged p = make_paged(kv_data, kv_param, kv_indptr, kv_indices, last_page_offset, num_layers,
+                         layer_idx, n_kv_heads, page_size, head_dim);
+    const int64_t blocks = srq_cdiv(batch * seq_len * (n_q_heads + 2 * n_kv_heads), 16);
+    SRQ_CHECK_ARG(blocks <= 0x7fffffffLL, "%s: too many rows", name);
+    prefill_qkv_kernel<<<dim3((unsigned)blocks), 256, 0, (hipStream_t)stream>>>(a, p);
     SRQ_LAUNCH_CHECK(name);
     return SRQ_OK;
 }

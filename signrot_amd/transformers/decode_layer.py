@@ -182,7 +182,12 @@ class W4A4LlamaDecodeLayer(torch.nn.Module):
         the cache (only the mask's 1-positions), the attention runs causal
         over the fp16 q/k/v (the flash-attn 2 call it replaces), then o_proj
         and the MLP as in decode.  Returns fp16 [B, T, hidden]; rows at
-        padding positions are computed but carry no meaning."""
+        padding positions are computed but carry no meaning.  With a dict
+        `trace` the intermediates are stored in it and the op-by-op path
+        runs; otherwise the fused kernels do where they have a form for the
+        sizes, with bit-identical results."""
+        if trace is None and self._prefill_fusable(hidden_states):
+            return self._prefill_fused(hidden_states, cache, cos, sin, attention_mask)
         B, T, _ = hidden_states.shape
         D, Hq, Hk = self.head_dim, self.n_heads, self.n_kv
         x2 = hidden_states.reshape(B * T, self.hidden)
@@ -205,6 +210,48 @@ class W4A4LlamaDecodeLayer(torch.nn.Module):
         keep("attn", attn)
         x2 = self._attn_out(attn.reshape(B * T, Hq, D), x2, keep)
         return self._mlp(x2, keep).view(B, T, self.hidden)
+
+    def _prefill_fusable(self, h):
+        """Sizes and alignment that rmsnorm_quant, head_had_quant and the
+        SwiGLU epilogue all take (head counts below 8 have no op-by-op
+        rotation either: hadamard_transform starts at 8)."""
+        return (h.dtype == torch.float16 and h.is_cuda and h.numel() > 0
+                and h.data_ptr() % 16 == 0 and self.hidden % 8 == 0 and self.hidden <= 8192
+                and self.ffn % 8 == 0 and 8 <= self.n_heads <= 64
+                and self.n_heads & (self.n_heads - 1) == 0)
+
+    def _prefill_fused(self, hidden_states, cache, cos, sin, attention_mask):
+        """rmsnorm_quant -> q/k/v GEMM -> prefill_qkv_cache (RoPE in place, K
+        Hadamard, KV quantize + cache fill; the op-by-op update when padding
+        has to be left out of the cache) -> prefill attention over the strided
+        views -> head_had_quant -> o_proj GEMM + residual -> rmsnorm_quant ->
+        gate/up GEMM with the SwiGLU in its epilogue -> had_sign_quant -> down
+        GEMM + residual."""
+        B, T, _ = hidden_states.shape
+        D, Hq, Hk = self.head_dim, self.n_heads, self.n_kv
+        x2 = hidden_states.reshape(B * T, self.hidden).contiguous()
+        n1, n2 = self.input_layernorm, self.post_attention_layernorm
+        q1, s1 = _CUDA.rmsnorm_quant(x2, n1.eps, n1.mean_dim)
+        qkv = _CUDA.w4a4_linear(q1, s1.view(-1), self.w_qkv, self.s_qkv)
+        if attention_mask is None:
+            q, k, v = cache.update_qkv_prefill(qkv.view(B, T, -1), cos, sin, self.layer_idx, Hq)
+        else:
+            heads = qkv.view(B, T, Hq + 2 * Hk, D).split((Hq, Hk, Hk), dim=2)
+            q, k, v = (t.contiguous() for t in heads)
+            kernel.rope_qk(q, k, cos, sin)
+            out = cache.update(k, v, self.layer_idx, {"attention_mask": attention_mask})
+            if not isinstance(out, tuple):
+                raise RuntimeError("prefill: the cache already holds this layer's context")
+            k, v = out
+        attn = _CUDA.prefill_attention(q, k, v, attention_mask, causal=True)
+        qa, sa = _CUDA.head_had_quant(attn.view(B * T, Hq, D), _inv_sqrt_f32(Hq))
+        x2 = _CUDA.w4a4_linear_residual(qa, sa.view(-1), self.w_o, self.s_o, x2)
+        q2, s2 = _CUDA.rmsnorm_quant(x2, n2.eps, n2.mean_dim)
+        w_il, s_il = self._gate_up_interleaved()
+        a = _CUDA.w4a4_linear_swiglu(q2, s2.view(-1), w_il, s_il)
+        qd, sd = _CUDA.had_sign_quant(a, self.down_hadk, self.down_k, self.down_sign)
+        out = _CUDA.w4a4_linear_residual(qd, sd.view(-1), self.w_down, self.s_down, x2, out=x2)
+        return out.view(B, T, self.hidden)
 
     @staticmethod
     def _keeper(trace):

@@ -418,6 +418,34 @@ class MultiLayerPagedKVCache4Bit(Cache):
                                          had_scale=1 / math.sqrt(self.head_dim),
                                          rotate=self.hadamard_dtype is not None)
 
+    def update_qkv_prefill(self, qkv, cos, sin, layer_idx, num_q_heads):
+        """First update of a layer from its q/k/v projection output qkv f16
+        [B, T, (Hq + 2 H) D] of a prompt without padding, one kernel: RoPE of
+        q and k (in place in qkv; cos/sin [1 or B, T, D]), k and v quantized
+        into the cache.  Returns views q [B, T, Hq, D], k and v [B, T, H, D]
+        of qkv for the prefill attention.  The cache bytes and q/k/v are those
+        of rope_qk and update() bit for bit."""
+        B, T = qkv.shape[:2]
+        if B != self.batch_size:
+            raise ValueError(f"batch {B} != the cache's {self.batch_size}")
+        if qkv.shape[2] != (num_q_heads + 2 * self.num_heads) * self.head_dim:
+            raise ValueError(f"update_qkv_prefill() takes {num_q_heads} query and "
+                             f"{self.num_heads} KV heads, got {qkv.shape[2]} columns")
+        if self._filled[layer_idx]:
+            if T != 1:
+                raise ValueError("after the prefill, update() appends one token per request")
+            raise RuntimeError("prefill: the cache already holds this layer's context")
+        if layer_idx == 0:
+            self._reserve(self.length + T)
+            self.length += T
+        spec = self.get_cache_specs_for_flash_infer(None)
+        self._filled[layer_idx] = True
+        _CUDA.prefill_qkv_cache(qkv, cos.contiguous(), sin.contiguous(), num_q_heads, **spec,
+                                layer_idx=layer_idx, had_scale=1 / math.sqrt(self.head_dim),
+                                rotate=self.hadamard_dtype is not None)
+        heads = qkv.view(B, T, num_q_heads + 2 * self.num_heads, self.head_dim)
+        return heads.split((num_q_heads, self.num_heads, self.num_heads), dim=2)
+
     def _qkv_step(self, qkv, layer_idx, attention_mask, name):
         if not self._filled[layer_idx]:
             raise RuntimeError(f"{name}: the layer has no prefill yet")

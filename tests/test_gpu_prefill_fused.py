@@ -1,0 +1,78 @@
+"""The fused prefill of the decoder layer against its op-by-op path (which
+test_gpu_prefill_layer.py checks against the oracle): the same hidden states
+and cache bytes, bit for bit, with and without padding, at the edges of pages
+and row blocks."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+D = 128
+
+
+def _layer(hidden, Hq, Hkv, ffn):
+    from signrot_amd.transformers.decode_layer import W4A4LlamaDecodeLayer
+    return W4A4LlamaDecodeLayer.random(hidden, Hq, Hkv, D, ffn, seed=5)
+
+
+def _cos_sin(B, T, per_request):
+    from signrot_amd.transformers.decode_layer import rope_cos_sin
+    if not per_request:
+        return rope_cos_sin(range(T), D, 500000.0, "cuda")
+    cs = [rope_cos_sin(range(3 * b, 3 * b + T), D, 500000.0, "cuda") for b in range(B)]
+    return torch.cat([c for c, _ in cs]), torch.cat([s for _, s in cs])
+
+
+def _run(layer, h, B, T, page, cos, sin, mask, trace):
+    from signrot_amd.transformers import MultiLayerPagedKVCache4Bit
+    cache = MultiLayerPagedKVCache4Bit(B, page, T, "cuda", 1, layer.n_kv, D,
+                                       group_size=layer.n_heads // layer.n_kv)
+    cache.pages.zero_()
+    cache.scales.zero_()
+    out = layer.prefill(h, cache, cos, sin, attention_mask=mask, trace=trace)
+    return out, cache.pages, cache.scales
+
+
+# heads whose rows split a wave between kinds (9 and 5 slots), one token, page
+# edges, more rows than rmsnorm's per-row form takes
+@pytest.mark.parametrize("B,T,Hq,Hkv,page", [(1, 1, 8, 2, 16), (3, 40, 8, 2, 32),
+                                             (2, 33, 8, 1, 16), (1, 300, 16, 4, 64),
+                                             (2, 64, 8, 8, 64)])
+@pytest.mark.parametrize("per_request", [False, True])
+def test_fused_prefill_bitexact(B, T, Hq, Hkv, page, per_request):
+    hidden = Hq * D
+    layer = _layer(hidden, Hq, Hkv, 896)
+    h = torch.randn(B, T, hidden, device="cuda", generator=torch.Generator("cuda").manual_seed(T))
+    h = h.half()
+    cos, sin = _cos_sin(B, T, per_request)
+    keep = h.clone()
+    fused = _run(layer, h, B, T, page, cos, sin, None, None)
+    ops = _run(layer, h, B, T, page, cos, sin, None, {})
+    assert torch.equal(h, keep)
+    for a, b, what in zip(fused, ops, ("hidden", "codes", "params")):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), what
+
+
+def test_fused_prefill_masked_bitexact():
+    B, T, page = 3, 40, 32
+    layer = _layer(1024, 8, 2, 896)
+    h = torch.randn(B, T, 1024, device="cuda").half()
+    lens = torch.tensor([40, 33, 36], device="cuda")
+    mask = (torch.arange(T, device="cuda")[None] >= (T - lens)[:, None]).int()
+    cos, sin = _cos_sin(B, T, False)
+    fused = _run(layer, h, B, T, page, cos, sin, mask, None)
+    ops = _run(layer, h, B, T, page, cos, sin, mask, {})
+    for a, b in zip(fused, ops):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+def test_fused_prefill_refuses_a_filled_layer():
+    from signrot_amd.transformers import MultiLayerPagedKVCache4Bit
+    layer = _layer(1024, 8, 2, 896)
+    cos, sin = _cos_sin(1, 8, False)
+    cache = MultiLayerPagedKVCache4Bit(1, 16, 16, "cuda", 1, 2, D, group_size=4)
+    h = torch.randn(1, 8, 1024, device="cuda").half()
+    layer.prefill(h, cache, cos, sin)
+    with pytest.raises(ValueError):
+        layer.prefill(h, cache, cos, sin)
+    assert cache.length == 8
