@@ -32,10 +32,12 @@ import torch
 from . import _native
 
 _call = _native.call
+_host = _native.host   # the same ops in C++ for arguments that need no second look
 
 
 def _stream(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    s = _host.stream(t)
+    return torch.cuda.current_stream(t.device).cuda_stream if s is None else s
 
 
 def _check(name, tensors, dtypes=None, contiguous=True):
@@ -97,6 +99,9 @@ def w4a4_linear_asym(A, a_scale, a_zero, B, b_scale, b_sum, bias=None):
     (int32) -> sym_dequant (+ bias); A uint4 codes [M, K/2], a_zero int8
     [M], b_sum int32 [N] (sum_i4 of B).  The zeros_x branch of
     Linear4bit.forward (linear.py:35-50) in one launch."""
+    out = _host.w4a4_linear_asym(A, a_scale, a_zero, B, b_scale, b_sum, bias, 2)
+    if out is not None:
+        return out
     _check("w4a4_linear_asym", [(A, "A"), (a_scale, "a_scale"), (a_zero, "a_zero"), (B, "B"),
                                 (b_scale, "b_scale"), (b_sum, "b_sum"), (bias, "bias")],
            [torch.uint8, torch.float16, torch.int8, torch.uint8, torch.float16, torch.int32,
@@ -119,6 +124,9 @@ def w4a4_linear_asym(A, a_scale, a_zero, B, b_scale, b_sum, bias=None):
 
 def w4a4_linear(A, a_scale, B, b_scale, bias=None):
     """Fused matmul + sym_dequant (+ fp16 bias): out f16 [M, N]."""
+    out = _host.w4a4_linear(A, a_scale, B, b_scale, bias, 2)
+    if out is not None:
+        return out
     _check("w4a4_linear", [(A, "A"), (a_scale, "a_scale"), (B, "B"), (b_scale, "b_scale"),
                            (bias, "bias")],
            [torch.uint8, torch.float16, torch.uint8, torch.float16, torch.float16])
@@ -158,6 +166,9 @@ def interleave_gate_up(w, s, ffn):
 def w4a4_linear_swiglu(A, a_scale, B_il, b_scale_il):
     """swiglu(gate, up) of the gate/up projection in one launch (any M):
     B_il / b_scale_il from interleave_gate_up; out f16 [M, N/2]."""
+    out = _host.w4a4_linear_swiglu(A, a_scale, B_il, b_scale_il)
+    if out is not None:
+        return out
     _check("w4a4_linear_swiglu", [(A, "A"), (a_scale, "a_scale"), (B_il, "B"),
                                   (b_scale_il, "b_scale")],
            [torch.uint8, torch.float16, torch.uint8, torch.float16])
@@ -259,6 +270,9 @@ def w4a4_linear_bf6(A6, a_scale, B6, b_scale, M, N, K, bias=None):
 def w4a4_linear_residual(A, a_scale, B, b_scale, residual, bias=None, out=None):
     """w4a4_linear with `+ residual` fused into the epilogue: out f16 [M, N] =
     fp16(linear + residual).  `out` may be `residual` itself (in place)."""
+    res = _host.w4a4_linear_residual(A, a_scale, B, b_scale, residual, bias, out)
+    if res is not None:
+        return res
     _check("w4a4_linear_residual", [(A, "A"), (a_scale, "a_scale"), (B, "B"),
                                     (b_scale, "b_scale"), (residual, "residual"), (bias, "bias"),
                                     (out, "out")],
@@ -328,6 +342,9 @@ def sym_dequant(q, scale_row, scale_col, bits=32):
 
 def sym_quant_dynamic(x, clip_ratio=1.0):
     """(q u8 [rows, ceil(cols/2)], scale f16 [rows, 1]) (bindings.cpp:316-335)."""
+    out = _host.sym_quant_dynamic(x, clip_ratio, 2)
+    if out is not None:
+        return out
     _check("sym_quant_dynamic", [(x, "x")])
     if x.dim() != 2:
         raise RuntimeError("sym_quant_dynamic expects a 2D [rows, cols] tensor")
@@ -474,6 +491,9 @@ def online_hadamard(x, hadK, K, sign=None, fp32_had=False):
 def had_sign_quant(x, hadK, K, sign=None, clip_ratio=1.0, fp32_had=False):
     """online_hadamard followed by sym_quant_dynamic, one launch:
     (q u8 [..., n/2], scale f16 [..., 1])."""
+    out = _host.had_sign_quant(x, hadK, K, sign, clip_ratio, fp32_had)
+    if out is not None:
+        return out
     _check("had_sign_quant", [(x, "x"), (hadK, "hadK"), (sign, "sign")],
            [torch.float16, None, torch.int8])
     n = x.shape[-1]
@@ -503,6 +523,9 @@ def had_sign_asym_quant(x, hadK, K, sign=None, clip_ratio=1.0):
     codes, scale f16 [..., 1], zero f16 [..., 1]).  One launch where the
     rotation has an MFMA form (had_asym_fusable), else the two ops in turn
     (the same results)."""
+    out = _host.had_sign_asym_quant(x, hadK, K, sign, clip_ratio)
+    if out is not None:
+        return out
     _check("had_sign_asym_quant", [(x, "x"), (hadK, "hadK"), (sign, "sign")],
            [torch.float16, torch.float16, torch.int8])
     n = x.shape[-1]
@@ -752,6 +775,10 @@ def rmsnorm(x, eps, mean_dim):
 def rmsnorm_quant(x, eps, mean_dim, clip_ratio=1.0, return_norm=False):
     """rmsnorm followed by sym_quant_dynamic in one launch: (q u8 [..., cols/2],
     scale f16 [..., 1]) and, with return_norm, the fp16 normalized x."""
+    if not return_norm:
+        out = _host.rmsnorm_quant(x, eps, mean_dim, clip_ratio)
+        if out is not None:
+            return out
     _check("rmsnorm_quant", [(x, "x")], [torch.float16])
     cols = x.shape[-1]
     rows = x.numel() // cols if cols else 0
@@ -789,6 +816,10 @@ def head_had_quant(x, scale, clip_ratio=1.0, return_rot=False):
     """Head-axis Hadamard of x f16 [B, H, D] (times `scale`) then per-row
     sym_quant_dynamic of the [B, H * D] result: (q u8 [B, H*D/2], scale f16
     [B, 1]) and, with return_rot, the rotated fp16 rows."""
+    if not return_rot:
+        out = _host.head_had_quant(x, scale, clip_ratio)
+        if out is not None:
+            return out
     _check("head_had_quant", [(x, "x")], [torch.float16])
     if x.dim() != 3:
         raise RuntimeError("head_had_quant expects x [B, H, D]")

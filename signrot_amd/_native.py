@@ -5,9 +5,12 @@ if the library is missing the import of the op table raises, so a GPU run
 can never silently use a CPU or PyTorch path instead of the HIP kernels.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import pathlib
 
 LIB_PATH = pathlib.Path(__file__).resolve().parent / "_lib" / "libsignrot_hip.so"
+HOST_PATH = LIB_PATH.with_name("srq_host.so")
 
 _i64 = ctypes.c_int64
 _i32 = ctypes.c_int
@@ -120,3 +123,25 @@ def call(name, *args):
     if rc != 0:
         msg = lib().srq_last_error().decode(errors="replace")
         raise NativeError(f"{name} failed ({rc}): {msg}")
+
+
+class _HostOps:
+    """The functions of srq_host.so (csrc/host.cpp), loaded on first use: each
+    runs one op for arguments that it takes as they stand and returns None for
+    any other, which the Python op then handles."""
+
+    def __getattr__(self, name):
+        lib()
+        if not HOST_PATH.exists():
+            raise RuntimeError(
+                f"signrot_amd: host extension not found at {HOST_PATH}; build it with "
+                "`python -m signrot_amd.csrc.build`")
+        loader = importlib.machinery.ExtensionFileLoader("srq_host", str(HOST_PATH))
+        spec = importlib.util.spec_from_loader("srq_host", loader)
+        mod = importlib.util.module_from_spec(spec)
+        loader.exec_module(mod)
+        self.__dict__.update({k: f for k, f in vars(mod).items() if not k.startswith("_")})
+        return self.__dict__[name]
+
+
+host = _HostOps()

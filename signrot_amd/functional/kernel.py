@@ -93,6 +93,9 @@ def matmul_si4_si4(A, B):
 
 def w4a4_linear(A, a_scale, B, b_scale, bias=None):
     """Fused matmul_si4_si4 + sym_dequant (+ bias): fp16 [..., N]."""
+    out = _CUDA._host.w4a4_linear(A, a_scale, B, b_scale, bias, 0)
+    if out is not None:
+        return out
     A, A_shape_excl_last = flatten_last_dim_and_return_shape(A)
     out = _CUDA.w4a4_linear(A, a_scale.reshape(-1), B, b_scale.reshape(-1),
                             None if bias is None else bias.reshape(-1))
@@ -111,6 +114,9 @@ def matmul_ui4_si4(A, B):
 def w4a4_linear_asym(A, a_scale, a_zero, B, b_scale, b_sum, bias=None):
     """Fused matmul_ui4_si4 - zeros ⊗ weight_sum + sym_dequant (+ bias):
     fp16 [..., N] (the zeros_x branch of Linear4bit.forward in one launch)."""
+    out = _CUDA._host.w4a4_linear_asym(A, a_scale, a_zero, B, b_scale, b_sum, bias, 0)
+    if out is not None:
+        return out
     A, A_shape_excl_last = flatten_last_dim_and_return_shape(A)
     out = _CUDA.w4a4_linear_asym(A, a_scale.reshape(-1), a_zero.reshape(-1), B,
                                  b_scale.reshape(-1), b_sum.reshape(-1),
@@ -180,6 +186,9 @@ def sym_quant_dynamic(x, clip_ratio=1.0):
     """Fused per-row amax + scale + symmetric int4 quantize/pack
     (kernel.py:101-110).  Returns (packed_q, scale) with scale shaped
     (*x.shape[:-1], 1)."""
+    out = _CUDA._host.sym_quant_dynamic(x, clip_ratio, 0)
+    if out is not None:
+        return out
     assert x.dtype == torch.float16
     x, shape_excl_last = flatten_last_dim_and_return_shape(x.contiguous())
     q, scale = _CUDA.sym_quant_dynamic(x, clip_ratio)
@@ -188,6 +197,9 @@ def sym_quant_dynamic(x, clip_ratio=1.0):
 
 def had_sign_quant(x, hadK, K, sign=None, clip_ratio=1.0, fp32_had=False):
     """Fused OnlineHadamard -> sign -> sym_quant_dynamic (one launch)."""
+    out = _CUDA._host.had_sign_quant(x, hadK, K, sign, clip_ratio, fp32_had)
+    if out is not None:
+        return out
     assert x.dtype == torch.float16
     x, shape_excl_last = flatten_last_dim_and_return_shape(x.contiguous())
     q, scale = _CUDA.had_sign_quant(x, hadK, K, sign, clip_ratio, fp32_had)

@@ -117,19 +117,18 @@ class HadamardQuantizer(torch.nn.Module):
         self.quantizer = quantizer
 
     def forward(self, x):
-        h = self.had
+        h, quantizer = self.had, self.quantizer
         if x.dtype != torch.float16 or not x.is_cuda:
-            return self.quantizer(h(x))
-        if isinstance(self.quantizer, AsymQuantizer):
+            return quantizer(h(x))
+        if isinstance(quantizer, AsymQuantizer):
             if h.fp32_had:
-                return self.quantizer(h(x))
+                return quantizer(h(x))
             q, s, z = _CUDA.had_sign_asym_quant(x.contiguous(), h._hadk(x.device), h.rem_dim,
-                                                h._sign(), self.quantizer.clip_ratio)
+                                                h._sign(), quantizer.clip_ratio)
             return kernel.PackedQuantizedTensor(q, s, z.to(torch.int8))
         q, s = kernel.had_sign_quant(x, h._hadk(x.device), h.rem_dim, h._sign(),
-                                     self.quantizer.clip_ratio, h.fp32_had)
+                                     quantizer.clip_ratio, h.fp32_had)
         return kernel.PackedQuantizedTensor(q, s)
-
 
 
 def fuse_online_hadamard(module: torch.nn.Module) -> torch.nn.Module:

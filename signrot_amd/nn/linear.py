@@ -58,7 +58,7 @@ class Linear4bit(torch.nn.Module):
         s = self.weight_scales
         if s.dtype != torch.float16:
             s = s.to(torch.float16)
-        return s.reshape(-1)
+        return s if s.is_contiguous() else s.reshape(-1)
 
     @staticmethod
     def from_float(module: torch.nn.Linear, weight_scales=None):
