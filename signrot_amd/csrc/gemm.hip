@@ -1875,6 +1875,199 @@ __global__ __launch_bounds__(64 * (4 + NPROD), 1) void gemm_grouped_kernel(Group
     }
 }
 
+// ---------------------------------------------------------------------------
+// Few rows per expert (decode batches): the grouped kernel's structure with
+// tiles of 32 FMB rows x 128 columns and a deeper ring that never drains.
+// With a handful of rows per expert the launch only has to stream the
+// experts' weights, but the 128-row form runs its MFMAs for 128 rows and has
+// two 16 KiB weight steps in flight per CU at most, fewer at each tile's end,
+// where its ring empties.  Here a stage holds 32 FMB + 128 rows, so NSTG = 7, 5 or 4
+// of them fit (FMB = 1, 2, 3), and the K steps of all tiles of a
+// workgroup form one sequence: the producers issue the next tile's steps
+// while the compute waves finish this one, so the epilogue (in LDS of its
+// own) is hidden and NSTG - 1 steps stay in flight throughout.  An expert
+// with more rows takes several row blocks, adjacent in the tile order so that
+// they read the same weights together.
+// Bound by HBM: gate/up of 8 experts (470 MB) in 100 us, 4.7 TB/s (figures at
+// moe_row_blocks).
+constexpr int kRowsBN = 128, kRowsKBB = 128;
+
+template <int FMB, bool UA, int FORM, int NSTG>
+__global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
+    constexpr int BM = 32 * FMB, KBB = kRowsKBB, NPROD = 4, kCompute = 4;
+    constexpr int kStage = (BM + kRowsBN) * KBB;
+    constexpr int C = KBB / 16, R = 1024 / KBB;    // chunks per row, rows per 1 KiB DMA
+    constexpr int kAPer = BM / R / NPROD, kBPer = kRowsBN / R / NPROD, kPer = kAPer + kBPer;
+    static_assert(kAPer * R * NPROD == BM && kBPer * R * NPROD == kRowsBN, "DMA split");
+    static_assert((NSTG - 2) * kPer <= 63, "vmcnt range");
+    constexpr int kEpiTile = 4 * 32 * BM;          // a compute wave's int32 block
+    static_assert(NSTG * kStage + kCompute * kEpiTile <= 160 * 1024, "LDS");
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[NSTG * kStage];
+    __shared__ __attribute__((aligned(16))) uint8_t epi_lds[kCompute * kEpiTile];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // tile walk, the same in every wave: t = blockIdx.x, + gridDim.x, ... of
+    // the experts' concatenated tile lists, row block fastest
+    int p = 0;
+    int64_t pstart = 0, t = blockIdx.x, m0 = 0, n0 = 0;
+    GroupedProb pr = grouped_prob<FORM>(g, 0);
+    auto tiles_of = [&]() -> int64_t {
+        return pr.m <= 0 ? 0 : srq_cdiv(pr.m, BM) * srq_cdiv(pr.n, kRowsBN);
+    };
+    int64_t ptiles = tiles_of();
+    auto locate = [&]() -> bool {
+        while (p < g.P && t >= pstart + ptiles) {
+            pstart += ptiles;
+            if (++p < g.P) {
+                pr = grouped_prob<FORM>(g, p);
+                ptiles = tiles_of();
+            }
+        }
+        if (p >= g.P) return false;
+        const int64_t tm = srq_cdiv(pr.m, BM), local = t - pstart;
+        m0 = local % tm * BM;
+        n0 = local / tm * kRowsBN;
+        return true;
+    };
+    const int64_t KB = g.K / 2;
+    const int steps = (int)((KB + KBB - 1) / KBB);
+    bool have = locate();
+
+    if (wave >= kCompute) {
+        const int pw = wave - kCompute;
+        const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)smem;
+        // DMA q of this wave: its A blocks, then its B blocks (8 rows each)
+        auto blk = [&](int q) {
+            return q < kAPer ? kAPer * pw + q : BM / R + kBPer * pw + (q - kAPer);
+        };
+        __amdgpu_buffer_rsrc_t ar, br;
+        uint32_t roff[kPer];
+        int jc[kPer];
+#pragma unroll
+        for (int q = 0; q < kPer; ++q)
+            jc[q] = ((lane % C) ^ swz<KBB>(R * blk(q) + lane / C)) * 16;
+        auto setup = [&]() {
+            ar = make_rsrc((const uint8_t *)uni((int64_t)pr.a), uni(pr.m * pr.lda_b));
+            br = make_rsrc((const uint8_t *)uni((int64_t)pr.b), uni(pr.n * pr.ldb_b));
+#pragma unroll
+            for (int q = 0; q < kPer; ++q) {
+                const int r = R * blk(q) + lane / C;
+                const int64_t row = q < kAPer ? m0 + r : n0 + r - BM;
+                roff[q] = row < (q < kAPer ? pr.m : pr.n) ? (uint32_t)(row * KB) : kOob;
+            }
+        };
+        int s = 0, issued = 0, slot = 0;
+        if (have) setup();
+        // the next step of the sequence into the next stage
+        auto issue = [&]() {
+            const int64_t kb0 = (int64_t)s * KBB;
+            const bool tail = kb0 + KBB > KB;
+#pragma unroll
+            for (int q = 0; q < kPer; ++q) {
+                uint32_t off = roff[q] == kOob ? kOob : roff[q] + (uint32_t)kb0 + jc[q];
+                if (tail && kb0 + jc[q] >= KB) off = kOob;
+                dma16(q < kAPer ? ar : br, off, lds0 + slot * kStage + blk(q) * 1024);
+            }
+            slot = slot == NSTG - 1 ? 0 : slot + 1;
+            ++issued;
+            if (++s == steps) {
+                s = 0;
+                t += gridDim.x;
+                have = locate();
+                if (have) setup();
+            }
+        };
+#pragma unroll 1
+        for (int q = 0; q < NSTG - 1 && have; ++q) issue();
+        for (int gs = 0; gs < issued; ++gs) {
+            // step gs of this wave is done (later ones may fly); after the
+            // barrier every wave's is, and the stage of step gs - 1 is free
+            ring_wait<kPer, NSTG - 2>(min(NSTG - 2, issued - gs - 1));
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            if (have) issue();
+        }
+        return;  // the compute waves meet no barrier after their last step
+    }
+
+    int slot = 0;
+    for (; have; t += gridDim.x, have = locate()) {
+        v16i acc[FMB][1];
+#pragma unroll
+        for (int i = 0; i < FMB; ++i) acc[i][0] = (v16i){};
+        for (int s = 0; s < steps; ++s) {
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            big_compute<FMB, 1, KBB, BM, UA>(smem + slot * kStage, 0, wave, lane, acc);
+            slot = slot == NSTG - 1 ? 0 : slot + 1;
+        }
+        const bool second = g.pair && (p & 1);
+        const int64_t ex = g.pair ? p >> 1 : p;
+        Epi e{};
+        e.out = (second ? g.out2 : g.out) + pr.row0 * (FORM == kFormSwiglu ? g.N / 2 : g.N);
+        e.sa = g.sa + pr.row0;
+        e.sb = (second ? g.sb2 : g.sb) + ex * g.N;
+        e.ua = UA;
+        if (g.zr) {
+            e.zr = g.zr + pr.row0;
+            e.ws = (second ? g.ws2 : g.ws) + ex * g.N;
+        }
+        int32_t *tile = reinterpret_cast<int32_t *>(epi_lds + wave * kEpiTile);
+        if constexpr (FORM == kFormSwiglu)
+            store_block_lds32_swiglu<32, FMB, 1>(e, pr.m, pr.n, m0, n0 + wave * 32, acc, lane, tile);
+        else
+            store_block_lds32<32, FMB, 1>(e, pr.m, pr.n, m0, n0 + wave * 32, acc, lane, tile);
+    }
+}
+
+// Row blocks (of 32) per tile of an expert-offset launch of `rows` rows over
+// `experts` experts (the rows of each are known on the device only): 1, 2 or
+// 3 on gemm_rows_kernel, 0 for the 128-row kernel.  The lines lie where most
+// experts still fit one row block of a router that is not far from even.
+// gate/up + SwiGLU / down of 8 experts (4096 / 14336) against the 128-row
+// kernel, us (one MI355X, two weight sets in turn):
+//   rows per expert     1           6           24          32          48          64
+//   128-row kernel  105 / 58   141 / 62    138 / 63    138 / 66    145 / 65    150 / 68
+//   1 block          73 / 37   100 / 52    101 / 52    119 / 72    152 / 76    195 / 105
+//   2 blocks         76 / 43   107 / 52    109 / 52    111 / 53    115 / 53    166 / 87
+//   3 blocks                                                       127 / 61    132 / 62
+// 80 rows per expert: 153 / 71 -> 139 / 64 with 3 blocks; 96: 161 / 72
+// against 193 / 98.
+int moe_row_blocks(int64_t rows, int64_t experts, int64_t K) {
+    if (K < 32) return 0;
+    if (rows <= 20 * experts) return 1;
+    if (rows <= 48 * experts) return 2;
+    if (rows <= 80 * experts) return 3;
+    return 0;
+}
+
+template <bool UA, int FORM>
+void launch_moe(const GroupedArgs &g, int64_t rows, hipStream_t st) {
+    switch (moe_row_blocks(rows, g.pair ? g.P / 2 : g.P, g.K)) {
+    case 1: {
+        GroupedArgs r = g;
+        r.skip_rem = 0;
+        gemm_rows_kernel<1, UA, FORM, 7><<<dim3(kGroupedGrid), dim3(512), 0, st>>>(r);
+        break;
+    }
+    case 2: {
+        GroupedArgs r = g;
+        r.skip_rem = 0;
+        gemm_rows_kernel<2, UA, FORM, 5><<<dim3(kGroupedGrid), dim3(512), 0, st>>>(r);
+        break;
+    }
+    case 3: {
+        GroupedArgs r = g;
+        r.skip_rem = 0;
+        gemm_rows_kernel<3, UA, FORM, 4><<<dim3(kGroupedGrid), dim3(512), 0, st>>>(r);
+        break;
+    }
+    default:
+        gemm_grouped_kernel<4, UA, FORM><<<dim3(kGroupedGrid), dim3(512), 0, st>>>(g);
+    }
+}
+
 int check_gemm(const char *name, const void *A, const void *B, int64_t M, int64_t N,
                int64_t K) {
     SRQ_CHECK_ARG(M >= 0 && N >= 0 && K >= 0, "%s: negative shape", name);
@@ -2358,7 +2551,7 @@ extern "C" int srq_w4a4_linear_moe(const void *A, const void *a_scale, const voi
     g.sb = (const f16 *)b_scale;
     g.out = (f16 *)out;
     g.skip_rem = K > 2 * kGrpKBB;  // at least two K steps (the extra rows' schedule)
-    gemm_grouped_kernel<4, false><<<dim3(kGroupedGrid), dim3(512), 0, (hipStream_t)stream>>>(g);
+    launch_moe<false, kFormGeneral>(g, rows, (hipStream_t)stream);
     SRQ_LAUNCH_CHECK("w4a4_linear_moe");
     return SRQ_OK;
 }
@@ -2393,8 +2586,7 @@ extern "C" int srq_w4a4_linear_moe_swiglu(const void *A, const void *a_scale, co
     g.sb = (const f16 *)b_scale;
     g.out = (f16 *)out;
     g.skip_rem = K > 2 * kGrpKBB;  // at least two K steps (the extra rows' schedule)
-    gemm_grouped_kernel<4, false, kFormSwiglu>
-        <<<dim3(kGroupedGrid), dim3(512), 0, (hipStream_t)stream>>>(g);
+    launch_moe<false, kFormSwiglu>(g, rows, (hipStream_t)stream);
     SRQ_LAUNCH_CHECK("w4a4_linear_moe_swiglu");
     return SRQ_OK;
 }
@@ -2432,7 +2624,7 @@ extern "C" int srq_w4a4_linear_moe_gate_up(const void *A, const void *a_scale,
     g.sb2 = (const f16 *)s_up;
     g.out = (f16 *)out_gate;
     g.out2 = (f16 *)out_up;
-    gemm_grouped_kernel<4, false><<<dim3(kGroupedGrid), dim3(512), 0, (hipStream_t)stream>>>(g);
+    launch_moe<false, kFormGeneral>(g, rows, (hipStream_t)stream);
     SRQ_LAUNCH_CHECK("w4a4_linear_moe_gate_up");
     return SRQ_OK;
 }
@@ -2467,7 +2659,7 @@ extern "C" int srq_w4a4_linear_moe_asym(const void *A, const void *a_scale, cons
     g.out = (f16 *)out;
     g.zr = a_zero;
     g.ws = b_sum;
-    gemm_grouped_kernel<4, true><<<dim3(kGroupedGrid), dim3(512), 0, (hipStream_t)stream>>>(g);
+    launch_moe<true, kFormGeneral>(g, rows, (hipStream_t)stream);
     SRQ_LAUNCH_CHECK("w4a4_linear_moe_asym");
     return SRQ_OK;
 }
