@@ -606,6 +606,8 @@ def gemm_kernel_name(M, N, K=None, split=False):
         return -(-a // b)
     if M <= 32:
         return "gemm_stream_kernel (srq_w4a4_linear)"
+    if 32 < M <= 96 and split:
+        return "gemm_rows_kernel split-K form + splitk_reduce_kernel (srq_w4a4_linear_ws)"
     if M <= 64:
         return "gemm_skinny_kernel (srq_w4a4_linear)"
     if M >= 1024 and cdiv(M, 256) * cdiv(N, 256) >= 256:

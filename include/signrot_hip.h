@@ -153,6 +153,15 @@ int srq_w4a4_linear_asym(const void *A, const void *a_scale, const int8_t *a_zer
                          const void *bias, int64_t M, int64_t N, int64_t K, void *out,
                          void *stream);
 
+/* srq_w4a4_linear_asym with a caller-owned workspace of
+ * srq_w4a4_linear_ws_bytes(M, N, K) bytes (16-byte aligned; null or smaller:
+ * the plain form): mid-size M with few output tiles is split over K into
+ * int32 partials.  Bit-identical to srq_w4a4_linear_asym. */
+int srq_w4a4_linear_asym_ws(const void *A, const void *a_scale, const int8_t *a_zero,
+                            const void *B, const void *b_scale, const int32_t *b_sum,
+                            const void *bias, int64_t M, int64_t N, int64_t K, void *out,
+                            void *ws, int64_t ws_bytes, void *stream);
+
 /* srq_w4a4_linear with the decoder's residual add fused into the epilogue:
  * out = fp16(lin + residual[m, n]) after the dequant (and bias), as torch's
  * fp16 `residual + linear(x)` rounds it.  residual f16 [M, N]; out may be the

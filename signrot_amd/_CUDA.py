@@ -117,8 +117,14 @@ def w4a4_linear_asym(A, a_scale, a_zero, B, b_scale, b_sum, bias=None):
     if bias is not None and bias.numel() != N:
         raise RuntimeError("w4a4_linear_asym: bias must have N elements")
     out = torch.empty((M, N), dtype=torch.float16, device=A.device)
-    _call("srq_w4a4_linear_asym", _ptr(A), _ptr(a_scale), _ptr(a_zero), _ptr(B), _ptr(b_scale),
-          _ptr(b_sum), _ptr(bias), M, N, K, _ptr(out), _stream(A))
+    ws = _splitk_workspace(M, N, K, A.device)
+    if ws is None:
+        _call("srq_w4a4_linear_asym", _ptr(A), _ptr(a_scale), _ptr(a_zero), _ptr(B),
+              _ptr(b_scale), _ptr(b_sum), _ptr(bias), M, N, K, _ptr(out), _stream(A))
+    else:
+        _call("srq_w4a4_linear_asym_ws", _ptr(A), _ptr(a_scale), _ptr(a_zero), _ptr(B),
+              _ptr(b_scale), _ptr(b_sum), _ptr(bias), M, N, K, _ptr(out), _ptr(ws), ws.numel(),
+              _stream(A))
     return out
 
 

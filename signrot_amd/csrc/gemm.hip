@@ -1876,12 +1876,13 @@ __global__ __launch_bounds__(64 * (4 + NPROD), 1) void gemm_grouped_kernel(Group
 }
 
 // ---------------------------------------------------------------------------
-// Few rows per expert (decode batches): the grouped kernel's structure with
+// Few rows per expert (decode batches), and dense products of 33 to 192 rows
+// (dense_rows, splitk_plan): the grouped kernel's structure with
 // tiles of 32 FMB rows x 128 columns and a deeper ring that never drains.
 // With a handful of rows per expert the launch only has to stream the
 // experts' weights, but the 128-row form runs its MFMAs for 128 rows and has
 // two 16 KiB weight steps in flight per CU at most, fewer at each tile's end,
-// where its ring empties.  Here a stage holds 32 FMB + 128 rows, so NSTG = 7, 5 or 4
+// where its ring empties.  Here a stage holds 32 FMB + 128 rows, so NSTG = 7, 6 or 5
 // of them fit (FMB = 1, 2, 3), and the K steps of all tiles of a
 // workgroup form one sequence: the producers issue the next tile's steps
 // while the compute waves finish this one, so the epilogue (in LDS of its
@@ -1900,7 +1901,7 @@ __global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
     constexpr int kAPer = BM / R / NPROD, kBPer = kRowsBN / R / NPROD, kPer = kAPer + kBPer;
     static_assert(kAPer * R * NPROD == BM && kBPer * R * NPROD == kRowsBN, "DMA split");
     static_assert((NSTG - 2) * kPer <= 63, "vmcnt range");
-    constexpr int kEpiTile = 4 * 32 * BM;          // a compute wave's int32 block
+    constexpr int kEpiTile = 4 * 32 * 32;          // a compute wave's int32 row block
     static_assert(NSTG * kStage + kCompute * kEpiTile <= 160 * 1024, "LDS");
     __shared__ __attribute__((aligned(1024))) uint8_t smem[NSTG * kStage];
     __shared__ __attribute__((aligned(16))) uint8_t epi_lds[kCompute * kEpiTile];
@@ -1930,9 +1931,15 @@ __global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
         n0 = local / tm * kRowsBN;
         return true;
     };
-    const int64_t KB = g.K / 2;
-    const int steps = (int)((KB + KBB - 1) / KBB);
-    bool have = locate();
+    int64_t KB = 0;
+    int steps = 0;
+    auto next_tile = [&]() -> bool {
+        if (!locate()) return false;
+        KB = pr.k / 2;
+        steps = (int)((KB + KBB - 1) / KBB);
+        return true;
+    };
+    bool have = next_tile();
 
     if (wave >= kCompute) {
         const int pw = wave - kCompute;
@@ -1954,7 +1961,7 @@ __global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
             for (int q = 0; q < kPer; ++q) {
                 const int r = R * blk(q) + lane / C;
                 const int64_t row = q < kAPer ? m0 + r : n0 + r - BM;
-                roff[q] = row < (q < kAPer ? pr.m : pr.n) ? (uint32_t)(row * KB) : kOob;
+                roff[q] = row < (q < kAPer ? pr.m : pr.n) ? (uint32_t)(row * pr.lda_b) : kOob;
             }
         };
         int s = 0, issued = 0, slot = 0;
@@ -1974,7 +1981,7 @@ __global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
             if (++s == steps) {
                 s = 0;
                 t += gridDim.x;
-                have = locate();
+                have = next_tile();
                 if (have) setup();
             }
         };
@@ -1992,7 +1999,7 @@ __global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
     }
 
     int slot = 0;
-    for (; have; t += gridDim.x, have = locate()) {
+    for (; have; t += gridDim.x, have = next_tile()) {
         v16i acc[FMB][1];
 #pragma unroll
         for (int i = 0; i < FMB; ++i) acc[i][0] = (v16i){};
@@ -2002,10 +2009,27 @@ __global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
             big_compute<FMB, 1, KBB, BM, UA>(smem + slot * kStage, 0, wave, lane, acc);
             slot = slot == NSTG - 1 ? 0 : slot + 1;
         }
-        const bool second = g.pair && (p & 1);
-        const int64_t ex = g.pair ? p >> 1 : p;
+        if constexpr (FORM == kFormSplitK) {
+            // int32 partials: lane holds column lane & 31 of the wave's 32,
+            // rows 8 (v / 4) + 4 (lane / 32) + v % 4 of each block
+            const int64_t gn = n0 + wave * 32 + (lane & 31);
+            if (gn < pr.n) {
+#pragma unroll
+                for (int i = 0; i < FMB; ++i)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const int64_t gm = m0 + 32 * i + frag_row<32>(v, lane);
+                        if (gm < pr.m) pr.c[gm * pr.ldc + gn] = acc[i][0][v] >> (UA ? 4 : 8);
+                    }
+            }
+            continue;
+        }
+        constexpr bool DENSE = FORM == kFormDense;
+        const bool second = !DENSE && g.pair && (p & 1);
+        const int64_t ex = DENSE ? 0 : g.pair ? p >> 1 : p;
+        const bool sw = FORM == kFormSwiglu || (DENSE && g.swiglu);
         Epi e{};
-        e.out = (second ? g.out2 : g.out) + pr.row0 * (FORM == kFormSwiglu ? g.N / 2 : g.N);
+        e.out = (second ? g.out2 : g.out) + pr.row0 * (sw ? g.N / 2 : g.N);
         e.sa = g.sa + pr.row0;
         e.sb = (second ? g.sb2 : g.sb) + ex * g.N;
         e.ua = UA;
@@ -2013,11 +2037,41 @@ __global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
             e.zr = g.zr + pr.row0;
             e.ws = (second ? g.ws2 : g.ws) + ex * g.N;
         }
+        if constexpr (DENSE) {
+            e.bias = g.bias;
+            e.res = g.res;
+            e.ldo = g.ldo;
+        }
+        // one row block at a time through the wave's LDS tile
         int32_t *tile = reinterpret_cast<int32_t *>(epi_lds + wave * kEpiTile);
-        if constexpr (FORM == kFormSwiglu)
-            store_block_lds32_swiglu<32, FMB, 1>(e, pr.m, pr.n, m0, n0 + wave * 32, acc, lane, tile);
-        else
-            store_block_lds32<32, FMB, 1>(e, pr.m, pr.n, m0, n0 + wave * 32, acc, lane, tile);
+#pragma unroll
+        for (int i = 0; i < FMB; ++i) {
+            const v16i one[1][1] = {{acc[i][0]}};
+            if (m0 + 32 * i >= pr.m) break;
+            if (sw)
+                store_block_lds32_swiglu<32, 1, 1>(e, pr.m, pr.n, m0 + 32 * i, n0 + wave * 32, one,
+                                                   lane, tile);
+            else
+                store_block_lds32<32, 1, 1>(e, pr.m, pr.n, m0 + 32 * i, n0 + wave * 32, one, lane,
+                                            tile);
+        }
+    }
+}
+
+// Launch of FMB = fmb row blocks, ring stages by what LDS holds.
+template <bool UA, int FORM>
+void launch_rows(const GroupedArgs &g, int fmb, int64_t tiles, hipStream_t st) {
+    const dim3 grid((unsigned)std::min<int64_t>(tiles, kGroupedGrid)), block(512);
+    if constexpr (FORM == kFormGeneral || FORM == kFormSwiglu) {
+        if (fmb == 1) gemm_rows_kernel<1, UA, FORM, 7><<<grid, block, 0, st>>>(g);
+        else if (fmb == 2) gemm_rows_kernel<2, UA, FORM, 6><<<grid, block, 0, st>>>(g);
+        else gemm_rows_kernel<3, UA, FORM, 5><<<grid, block, 0, st>>>(g);
+    } else {
+        if (fmb <= 2) gemm_rows_kernel<2, UA, FORM, 6><<<grid, block, 0, st>>>(g);
+        else if (fmb == 3) gemm_rows_kernel<3, UA, FORM, 5><<<grid, block, 0, st>>>(g);
+        else if (fmb == 4) gemm_rows_kernel<4, UA, FORM, 4><<<grid, block, 0, st>>>(g);
+        else if (fmb == 5) gemm_rows_kernel<5, UA, FORM, 4><<<grid, block, 0, st>>>(g);
+        else gemm_rows_kernel<6, UA, FORM, 3><<<grid, block, 0, st>>>(g);
     }
 }
 
@@ -2044,26 +2098,12 @@ int moe_row_blocks(int64_t rows, int64_t experts, int64_t K) {
 
 template <bool UA, int FORM>
 void launch_moe(const GroupedArgs &g, int64_t rows, hipStream_t st) {
-    switch (moe_row_blocks(rows, g.pair ? g.P / 2 : g.P, g.K)) {
-    case 1: {
+    const int fmb = moe_row_blocks(rows, g.pair ? g.P / 2 : g.P, g.K);
+    if (fmb) {
         GroupedArgs r = g;
         r.skip_rem = 0;
-        gemm_rows_kernel<1, UA, FORM, 7><<<dim3(kGroupedGrid), dim3(512), 0, st>>>(r);
-        break;
-    }
-    case 2: {
-        GroupedArgs r = g;
-        r.skip_rem = 0;
-        gemm_rows_kernel<2, UA, FORM, 5><<<dim3(kGroupedGrid), dim3(512), 0, st>>>(r);
-        break;
-    }
-    case 3: {
-        GroupedArgs r = g;
-        r.skip_rem = 0;
-        gemm_rows_kernel<3, UA, FORM, 4><<<dim3(kGroupedGrid), dim3(512), 0, st>>>(r);
-        break;
-    }
-    default:
+        launch_rows<UA, FORM>(r, fmb, kGroupedGrid, st);
+    } else {
         gemm_grouped_kernel<4, UA, FORM><<<dim3(kGroupedGrid), dim3(512), 0, st>>>(g);
     }
 }
@@ -2167,13 +2207,55 @@ struct SplitK {
     int S = 0;
     int64_t Kc = 0;
     bool big = false;  // the big kernel's 256 x 128 tiles, grid (tiles, S)
+    bool rows = false; // gemm_rows_kernel, all M rows in one tile
 };
+
+// Dense products of 32 < M <= 192 rows whose 128-column tiles, all rows in one
+// tile, about cover the CUs: gemm_rows_kernel without a split (its weights
+// stream once, no rows are padded to 128).  us against the kernel that the
+// shape had (one MI355X), N = 28672, K = 4096: M = 33 / 64 / 96 / 137 / 192
+// 31 / 47 / 24 / 42 / 45 -> 18 / 19 / 24 / 31 / 35; with the SwiGLU epilogue
+// 21 / 22 / 22 / 38 / 40 -> 18 / 18 / 21 / 27 / 31; SwiGLU over N = 14336, M =
+// 64 / 128: 20 / 39 -> 16 / 22.  Between 97 and 128 rows the 128-row tiles
+// waste nothing (24.5 against 27.3), and past 128 rows fewer than 160 tiles
+// lose to the ring kernel (SwiGLU over 14336, M = 140: 21 against 25).
+bool dense_rows(int64_t M, int64_t N, int64_t K, bool swiglu) {
+    if (M <= 32 || M > 192 || K < 256) return false;
+    const int64_t ct = srq_cdiv(N, kRowsBN);
+    if (M <= 96) return ct >= (swiglu ? 96 : 192);
+    if (M <= 128) return swiglu && ct >= 96 && ct < 192;
+    return ct >= (swiglu ? 160 : 192);
+}
 SplitK splitk_plan(int64_t M, int64_t N, int64_t K, bool fp16_out) {
     SplitK p;
-    if (!fp16_out || M <= 64 || M >= 1024 || K < 2048) return p;
+    if (!fp16_out || M <= 32 || M >= 1024 || K < 2048) return p;
+    // Few column tiles: all rows in one gemm_rows_kernel tile, K in S chunks
+    // that give 160 to 256 tiles.  Up to 96 rows with chunks of at least 1280
+    // codes, M = 33 / 64 / 96: N = 4096, K = 14336 22 / 24 / 20.6 -> 15.6 / 17 /
+    // 19.8 us; N = 8192, K = 28672 67 / 75 / 44 -> 31 / 36 / 42 (N = 4096 or
+    // 6144 at K = 4096 lose: 8 against 12, 11.2 against 12.6).  Between 129
+    // and 192 rows only long chunks pay for the wider partials: M = 137 / 180
+    // at N = 8192, K = 28672 67 / 68 -> 55 / 58, but at N = 4096, K = 14336
+    // 24.6 / 25.6 against 24.8 / 27.3.
+    if (!dense_rows(M, N, K, false) && (M <= 96 || (M > 128 && M <= 192))) {
+        const int64_t ct = srq_cdiv(N, kRowsBN);
+        const int64_t S = std::min<int64_t>(256 / ct, K / (M <= 96 ? 1280 : 4096));
+        if (S >= 2 && ct * S >= 160) {
+            p.Kc = srq_cdiv(srq_cdiv(K, S), 256) * 256;
+            p.S = (int)srq_cdiv(K, p.Kc);
+            p.rows = true;
+            return p;
+        }
+    }
+    if (M <= 64) return p;
     const int64_t tiles = srq_cdiv(M, kGrpBM) * srq_cdiv(N, kGrpBN);
     const int64_t big = srq_cdiv(M, kBigBM) * srq_cdiv(N, kBigBN);
-    if (tiles >= 192 && big >= 64 && big <= 128 && 256 % big == 0 && K / (256 / big) >= 4096) {
+    // Past M = 512 only with chunks of 12288 codes: M = 1000 / 800, N = 4096, K =
+    // 14336 (two chunks of 7168) 57.7 / 54.1 us unsplit on the dense grouped
+    // form against 62.9 / 59.1 split; M = 512, N = 8192, K = 28672 112 against
+    // 106.
+    if (tiles >= 192 && big >= 64 && big <= 128 && 256 % big == 0 &&
+        K / (256 / big) >= (M <= 512 ? 4096 : 12288)) {
         // enough 128 x 128 tiles for the dense grouped form, but 256 / big
         // K-chunks of 256 x 128 tiles cover the CUs exactly, and the bigger
         // tile unpacks fewer nibbles per MFMA (the grouped kernel's compute
@@ -2214,6 +2296,28 @@ void splitk_reduce(const void *ws, int S, int64_t M, int64_t N, const Epi &e, hi
     }
 }
 
+// One dense problem with e's fp16 epilogue.
+GroupedArgs dense_args(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K,
+                       const Epi &e) {
+    GroupedArgs g{};
+    g.P = 1;
+    g.M = M;
+    g.A = a;
+    g.B = b;
+    g.N = N;
+    g.K = K;
+    g.sa = e.sa;
+    g.sb = e.sb;
+    g.out = e.out;
+    g.bias = e.bias;
+    g.res = e.res;
+    g.zr = e.zr;
+    g.ws = e.ws;
+    g.swiglu = e.swiglu;
+    g.ldo = e.ldo;
+    return g;
+}
+
 // Kernel choice by shape; UA: A holds unsigned nibbles (Epi::ua).  With a
 // workspace of at least splitk_bytes, mid-size M shapes with few tiles run
 // split over K.
@@ -2226,6 +2330,16 @@ void launch_gemm(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64
         fill_zero_epilogue<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(M, N, e);
     } else if (launch_stream<UA>(a, b, M, N, K, e, st)) {
         // M <= 32: persistent weight-streaming kernel
+    } else if (!e.C && dense_rows(M, N, K, e.swiglu != 0)) {
+        GroupedArgs g = dense_args(a, b, M, N, K, e);
+        launch_rows<UA, kFormDense>(g, (int)srq_cdiv(M, 32), srq_cdiv(N, kRowsBN), st);
+    } else if (sk.S && sk.rows && !e.swiglu && ws_bytes >= (int64_t)sk.S * M * N * 4) {
+        GroupedArgs g = dense_args(a, b, M, N, K, Epi{});
+        g.P = sk.S;
+        g.Kc = sk.Kc;
+        g.ws_c = (int32_t *)ws;
+        launch_rows<UA, kFormSplitK>(g, (int)srq_cdiv(M, 32), srq_cdiv(N, kRowsBN) * sk.S, st);
+        splitk_reduce(ws, sk.S, M, N, e, st);
     } else if (M <= 16 && !e.swiglu) {
         gemm_skinny_kernel<1, 8, 4, UA><<<dim3((unsigned)srq_cdiv(N, 16), 1), dim3(512), 0, st>>>(
             a, b, M, N, K, e);
@@ -2250,16 +2364,11 @@ void launch_gemm(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64
         gemm_big_kernel<4, 2, 2, 4, 2, 128, 3, UA>
             <<<dim3((unsigned)tiles, (unsigned)sk.S), dim3(512), 0, st>>>(a, b, M, N, K, ep, sk.Kc);
         splitk_reduce(ws, sk.S, M, N, e, st);
-    } else if (sk.S && !e.swiglu && ws_bytes >= (int64_t)sk.S * M * N * 4) {
+    } else if (sk.S && !sk.rows && !e.swiglu && ws_bytes >= (int64_t)sk.S * M * N * 4) {
         // split-K: S dense problems over K-chunks write int32 partials,
         // then one pass sums them and runs the epilogue
-        GroupedArgs g{};
+        GroupedArgs g = dense_args(a, b, M, N, K, Epi{});
         g.P = sk.S;
-        g.M = M;
-        g.A = a;
-        g.B = b;
-        g.N = N;
-        g.K = K;
         g.Kc = sk.Kc;
         g.ws_c = (int32_t *)ws;
         const int64_t tiles = srq_cdiv(M, kGrpBM) * srq_cdiv(N, kGrpBN) * sk.S;
@@ -2272,22 +2381,7 @@ void launch_gemm(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64
         // kernel's dense form (64 x 64 32x32-MFMA tiles per compute wave,
         // MFMA-bound where the ring kernel's small tiles are bound by the
         // nibble unpacking: 188 -> 113 us at M = 512, N = 8192, K = 28672)
-        GroupedArgs g{};
-        g.P = 1;
-        g.M = M;
-        g.A = a;
-        g.B = b;
-        g.N = N;
-        g.K = K;
-        g.sa = e.sa;
-        g.sb = e.sb;
-        g.out = e.out;
-        g.bias = e.bias;
-        g.res = e.res;
-        g.zr = e.zr;
-        g.ws = e.ws;
-        g.swiglu = e.swiglu;
-        g.ldo = e.ldo;
+        const GroupedArgs g = dense_args(a, b, M, N, K, e);
         const int64_t tiles = srq_cdiv(M, kGrpBM) * srq_cdiv(N, kGrpBN);
         gemm_grouped_kernel<4, UA, kFormDense>
             <<<dim3((unsigned)std::min<int64_t>(tiles, kGroupedGrid)), dim3(512), 0, st>>>(g);
@@ -2389,6 +2483,28 @@ extern "C" int srq_w4a4_linear_asym(const void *A, const void *a_scale, const in
     e.zr = a_zero;
     e.ws = b_sum;
     return run_gemm("w4a4_linear_asym", A, B, M, N, K, e, (hipStream_t)stream);
+}
+
+extern "C" int srq_w4a4_linear_asym_ws(const void *A, const void *a_scale, const int8_t *a_zero,
+                                       const void *B, const void *b_scale, const int32_t *b_sum,
+                                       const void *bias, int64_t M, int64_t N, int64_t K,
+                                       void *out, void *ws, int64_t ws_bytes, void *stream) {
+    int rc = check_gemm("w4a4_linear_asym_ws", A, B, M, N, K);
+    if (rc) return rc;
+    if (M && N)
+        SRQ_CHECK_ARG(out && a_scale && a_zero && b_scale && b_sum,
+                      "w4a4_linear_asym_ws: null pointer");
+    SRQ_CHECK_ARG(!ws || srq_aligned(ws, 16),
+                  "w4a4_linear_asym_ws: workspace must be 16-byte aligned");
+    Epi e{};
+    e.out = (f16 *)out;
+    e.sa = (const f16 *)a_scale;
+    e.sb = (const f16 *)b_scale;
+    e.bias = (const f16 *)bias;
+    e.ua = 1;
+    e.zr = a_zero;
+    e.ws = b_sum;
+    return run_gemm("w4a4_linear_asym_ws", A, B, M, N, K, e, (hipStream_t)stream, ws, ws_bytes);
 }
 
 extern "C" int srq_w4a4_linear(const void *A, const void *a_scale, const void *B,

@@ -343,14 +343,18 @@ PyObject *w4a4_linear_asym(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
         void *sa = ptr(a[1], kF16, o.M, o.dev), *za = ptr(a[2], kI8, o.M, o.dev);
         void *sb = ptr(a[4], kF16, o.N, o.dev), *wsum = ptr(a[5], kI32, o.N, o.dev);
         void *bias = opt_ptr(a[6], kF16, o.N, o.dev);
-        at::Tensor out;
+        at::Tensor out, ws;
         int rc;
         {
             NoGil nogil;
             out = alloc(with_last(o.A, o.N), kF16, o.dev);
-            rc = srq_w4a4_linear_asym(o.A.data_ptr(), sa, (const int8_t *)za, o.B.data_ptr(), sb,
-                                      (const int32_t *)wsum, bias, o.M, o.N, o.K,
-                                      out.data_ptr(), stream_of(o.dev));
+            const int64_t wb = srq_w4a4_linear_ws_bytes(o.M, o.N, o.K);
+            if (wb > 0) ws = alloc({wb}, kU8, o.dev);
+            rc = srq_w4a4_linear_asym_ws(o.A.data_ptr(), sa, (const int8_t *)za, o.B.data_ptr(),
+                                         sb, (const int32_t *)wsum, bias, o.M, o.N, o.K,
+                                         out.data_ptr(), wb > 0 ? ws.data_ptr() : nullptr,
+                                         wb > 0 ? wb : 0, stream_of(o.dev));
+            ws.reset();
         }
         if (rc) throw Bad();
         return wrap({out});
