@@ -268,6 +268,12 @@ int srq_had_sign_asym_quant(const void *x, int64_t rows, int64_t n, int64_t K,
                             const void *hadK, const int8_t *sign, float clip_ratio, void *q,
                             void *scale, void *zero, void *stream);
 
+/* srq_had_sign_asym_quant with the zero points as int8 [rows], the cast that
+ * AsymQuantizer makes of them (float to int, low byte). */
+int srq_had_sign_asym_quant_i8(const void *x, int64_t rows, int64_t n, int64_t K,
+                               const void *hadK, const int8_t *sign, float clip_ratio, void *q,
+                               void *scale, int8_t *zero, void *stream);
+
 /* srq_had_sign_quant whose input row is SwiGLU of two strided rows:
  * x[r, i] = fp16(fp16(silu(gate[r*ld + i])) * up[r*ld + i]) (the srq_swiglu
  * arithmetic), then the rotation, sign and quantizer of srq_had_sign_quant.
@@ -524,6 +530,12 @@ int srq_asym_quant_dynamic_moe(const void *x, const int8_t *sign, const int32_t 
                                int64_t num_experts, int64_t rows, int64_t cols,
                                float clip_ratio, void *q, void *scale, void *zero,
                                void *stream);
+
+/* srq_asym_quant_dynamic (sign NULL) or srq_asym_quant_dynamic_moe with the
+ * zero points as int8 [rows], the cast that AsymQuantizer makes of them. */
+int srq_asym_quant_dynamic_i8(const void *x, const int8_t *sign, const int32_t *expert_ids,
+                              int64_t num_experts, int64_t rows, int64_t cols, float clip_ratio,
+                              void *q, void *scale, int8_t *zero, void *stream);
 
 /* Asymmetric quantizer with a given per-row scale and zero (f16 [rows]):
  * q = clamp(__half2int_rn(fp16(x / scale)) + __half2int_rn(zero), lo, hi)

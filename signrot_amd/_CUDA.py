@@ -382,9 +382,10 @@ def sym_quant_dynamic_rows(x, src_row, clip_ratio=1.0):
 
 # ------------------------------------------------- asymmetric activations
 
-def asym_quant_dynamic(x, clip_ratio=1.0):
+def asym_quant_dynamic(x, clip_ratio=1.0, int8_zero=False):
     """(q u8 [rows, ceil(cols/2)] of uint4 codes, scale f16 [rows, 1], zero
-    f16 [rows, 1]) (bindings.cpp:337-358)."""
+    f16 [rows, 1]) (bindings.cpp:337-358).  int8_zero: zero.to(int8), the
+    form the GEMM takes, in the same launch."""
     _check("asym_quant_dynamic", [(x, "x")])
     if x.dim() != 2:
         raise RuntimeError("asym_quant_dynamic expects a 2D [rows, cols] tensor")
@@ -393,6 +394,11 @@ def asym_quant_dynamic(x, clip_ratio=1.0):
     rows, cols = x.shape
     q = torch.empty((rows, (cols + 1) // 2), dtype=torch.uint8, device=x.device)
     scale = torch.empty((rows, 1), dtype=torch.float16, device=x.device)
+    if int8_zero:
+        zero = torch.empty((rows, 1), dtype=torch.int8, device=x.device)
+        _call("srq_asym_quant_dynamic_i8", _ptr(x), None, None, 0, rows, cols,
+              float(clip_ratio), _ptr(q), _ptr(scale), _ptr(zero), _stream(x))
+        return q, scale, zero
     zero = torch.empty((rows, 1), dtype=torch.float16, device=x.device)
     _call("srq_asym_quant_dynamic", _ptr(x), rows, cols, float(clip_ratio), _ptr(q),
           _ptr(scale), _ptr(zero), _stream(x))
@@ -524,12 +530,12 @@ def had_asym_fusable(n, K):
         (n == K * 256 and K <= 64) or (n == K * 512 and 32 < K <= 64)
 
 
-def had_sign_asym_quant(x, hadK, K, sign=None, clip_ratio=1.0):
+def had_sign_asym_quant(x, hadK, K, sign=None, clip_ratio=1.0, int8_zero=False):
     """online_hadamard followed by asym_quant_dynamic: (q u8 [..., n/2] uint4
-    codes, scale f16 [..., 1], zero f16 [..., 1]).  One launch where the
-    rotation has an MFMA form (had_asym_fusable), else the two ops in turn
-    (the same results)."""
-    out = _host.had_sign_asym_quant(x, hadK, K, sign, clip_ratio)
+    codes, scale f16 [..., 1], zero f16 [..., 1], with int8_zero as int8).
+    One launch where the rotation has an MFMA form (had_asym_fusable), else
+    the two ops in turn (the same results)."""
+    out = _host.had_sign_asym_quant(x, hadK, K, sign, clip_ratio, int8_zero)
     if out is not None:
         return out
     _check("had_sign_asym_quant", [(x, "x"), (hadK, "hadK"), (sign, "sign")],
@@ -539,14 +545,15 @@ def had_sign_asym_quant(x, hadK, K, sign=None, clip_ratio=1.0):
     rows = x.numel() // n if n else 0
     if not had_asym_fusable(n, K) or hadK.data_ptr() % 8:
         rot = online_hadamard(x.reshape(rows, n), hadK, K, sign)
-        q, s, z = asym_quant_dynamic(rot, clip_ratio)
+        q, s, z = asym_quant_dynamic(rot, clip_ratio, int8_zero)
         return (q.view(*x.shape[:-1], -1), s.view(*x.shape[:-1], 1),
                 z.view(*x.shape[:-1], 1))
     q = torch.empty((*x.shape[:-1], n // 2), dtype=torch.uint8, device=x.device)
     scale = torch.empty((*x.shape[:-1], 1), dtype=torch.float16, device=x.device)
-    zero = torch.empty((*x.shape[:-1], 1), dtype=torch.float16, device=x.device)
+    zero = torch.empty((*x.shape[:-1], 1), dtype=torch.int8 if int8_zero else torch.float16,
+                       device=x.device)
     if rows:
-        _call("srq_had_sign_asym_quant", _ptr(x), rows, n, int(K), _ptr(hadK), _ptr(sign),
+        _call("srq_had_sign_asym_quant_i8" if int8_zero else "srq_had_sign_asym_quant", _ptr(x), rows, n, int(K), _ptr(hadK), _ptr(sign),
               float(clip_ratio), _ptr(q), _ptr(scale), _ptr(zero), _stream(x))
     return q, scale, zero
 
@@ -1027,10 +1034,10 @@ def swiglu_had_sign_quant_moe(gate, up, hadK, K, sign, expert_ids, clip_ratio=1.
     return q, scale
 
 
-def asym_quant_dynamic_moe(x, sign, expert_ids, clip_ratio=1.0):
+def asym_quant_dynamic_moe(x, sign, expert_ids, clip_ratio=1.0, int8_zero=False):
     """asym_quant_dynamic of expert-sorted rows with the per-expert sign fused
     (bindings.cpp:134-159).  Returns (q u8 [rows, ceil(cols/2)] uint4 codes,
-    scale f16 [rows, 1], zero f16 [rows, 1])."""
+    scale f16 [rows, 1], zero f16 [rows, 1], with int8_zero as int8)."""
     name = "asym_quant_dynamic_moe"
     _check(name, [(x, "x"), (expert_ids, "expert_ids")])
     if x.dim() != 2 or x.dtype != torch.float16:
@@ -1042,9 +1049,11 @@ def asym_quant_dynamic_moe(x, sign, expert_ids, clip_ratio=1.0):
     E = sign.shape[0] if sign is not None else 0
     q = torch.empty((rows, (cols + 1) // 2), dtype=torch.uint8, device=x.device)
     scale = torch.empty((rows, 1), dtype=torch.float16, device=x.device)
-    zero = torch.empty((rows, 1), dtype=torch.float16, device=x.device)
-    _call("srq_asym_quant_dynamic_moe", _ptr(x), _ptr(sign), _ptr(expert_ids), E, rows, cols,
-          float(clip_ratio), _ptr(q), _ptr(scale), _ptr(zero), _stream(x))
+    zero = torch.empty((rows, 1), dtype=torch.int8 if int8_zero else torch.float16,
+                       device=x.device)
+    _call("srq_asym_quant_dynamic_i8" if int8_zero else "srq_asym_quant_dynamic_moe", _ptr(x),
+          _ptr(sign), _ptr(expert_ids), E, rows, cols, float(clip_ratio), _ptr(q), _ptr(scale),
+          _ptr(zero), _stream(x))
     return q, scale, zero
 
 

@@ -37,6 +37,8 @@ SIGNATURES = {
                                 _p],
     "srq_w4a4_linear_moe_asym": [_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _p, _p],
     "srq_had_sign_asym_quant": [_p, _i64, _i64, _i64, _p, _p, _f32, _p, _p, _p, _p],
+    "srq_had_sign_asym_quant_i8": [_p, _i64, _i64, _i64, _p, _p, _f32, _p, _p, _p, _p],
+    "srq_asym_quant_dynamic_i8": [_p, _p, _p, _i64, _i64, _i64, _f32, _p, _p, _p, _p],
     "srq_asym_quant_dynamic": [_p, _i64, _i64, _f32, _p, _p, _p, _p],
     "srq_asym_quant_dynamic_moe": [_p, _p, _p, _i64, _i64, _i64, _f32, _p, _p, _p, _p],
     "srq_asym_quant": [_p, _p, _p, _i64, _i64, _i32, _p, _p],

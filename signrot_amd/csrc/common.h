@@ -219,6 +219,15 @@ SRQ_DEV void asym_row_params(float vmin, float vmax, float clip, f16 &scale, f16
     zero = f16_rn(__builtin_rintf((float)ratio));
 }
 
+// The zero point as int8, the GEMM's form: what torch's fp16 -> int8 cast
+// gives (float to int32, saturating, NaN -> 0, then the low byte).
+SRQ_DEV int8_t zero_i8(f16 z) {
+    const float f = (float)z;
+    int i;
+    asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(f));
+    return (int8_t)i;
+}
+
 // Asymmetric code: clamp(__half2int_rn(fp16(x / s)) + zero_i, lo, hi), the
 // quotient correctly rounded (fp32 division, then one fp16 rounding) and the
 // int addition wrapping in int32 as the reference's does.

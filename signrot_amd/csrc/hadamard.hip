@@ -406,11 +406,11 @@ int srq_had512_mfma(const void *x, int64_t rows, int64_t n, int64_t K, const voi
                     const int8_t *sign, float clip, void *q, void *qscale, void *out,
                     hipStream_t st, const void *up = nullptr, int64_t ld = 0,
                     const int32_t *sign_row = nullptr, int64_t n_sign_rows = 0,
-                    void *qzero = nullptr, int bf6 = 0);
+                    void *qzero = nullptr, int bf6 = 0, int8_t *qzero8 = nullptr);
 
 int srq_had_kron_mfma(const void *x, int64_t rows, int64_t n, int64_t K, const void *hadK,
                       const int8_t *sign, float clip, void *q, void *qscale, void *qzero,
-                      void *out, hipStream_t st);
+                      int8_t *qzero8, void *out, hipStream_t st);
 
 // Rotation + sign + quantizer of rows of n = 256 E (a power of two, K = 1:
 // the plain FWHT) for the decode-sized row counts of a q/k/v-shaped
@@ -601,8 +601,8 @@ extern "C" int srq_online_hadamard(const void *x, void *out, int64_t rows, int64
     if (!fp32_had &&
         (srq_had512_mfma(x, rows, n, K, hadK, sign, 1.f, nullptr, nullptr, out,
                          (hipStream_t)stream) ||
-         srq_had_kron_mfma(x, rows, n, K, hadK, sign, 1.f, nullptr, nullptr, nullptr, out,
-                           (hipStream_t)stream))) {
+         srq_had_kron_mfma(x, rows, n, K, hadK, sign, 1.f, nullptr, nullptr, nullptr, nullptr,
+                           out, (hipStream_t)stream))) {
         SRQ_LAUNCH_CHECK("online_hadamard");
         return SRQ_OK;
     }
@@ -635,7 +635,7 @@ extern "C" int srq_had_sign_quant(const void *x, int64_t rows, int64_t n, int64_
     if (!fp32_had && (srq_had512_mfma(x, rows, n, K, hadK, sign, clip_ratio, q, scale, nullptr,
                                       (hipStream_t)stream) ||
                       srq_had_kron_mfma(x, rows, n, K, hadK, sign, clip_ratio, q, scale, nullptr,
-                                        nullptr, (hipStream_t)stream))) {
+                                        nullptr, nullptr, (hipStream_t)stream))) {
         SRQ_LAUNCH_CHECK("had_sign_quant");
         return SRQ_OK;
     }
@@ -742,23 +742,36 @@ extern "C" int srq_had_sign_quant_bf6(const void *x, int64_t rows, int64_t n, in
     return SRQ_EUNSUPPORTED;
 }
 
+static int had_sign_asym(const char *name, const void *x, int64_t rows, int64_t n, int64_t K,
+                         const void *hadK, const int8_t *sign, float clip_ratio, void *q,
+                         void *scale, void *zero, int8_t *zero8, void *stream) {
+    int rc = check_rotation(name, x, rows, n, K, hadK);
+    if (rc) return rc;
+    if (rows == 0) return SRQ_OK;
+    SRQ_CHECK_ARG(q && scale && (zero || zero8), "%s: null output", name);
+    SRQ_CHECK_ARG(srq_aligned(x, 16) && srq_aligned(q, 16),
+                  "%s: x and q must be 16-byte aligned", name);
+    if (srq_had512_mfma(x, rows, n, K, hadK, sign, clip_ratio, q, scale, nullptr,
+                        (hipStream_t)stream, nullptr, 0, nullptr, 0, zero, 0, zero8) ||
+        srq_had_kron_mfma(x, rows, n, K, hadK, sign, clip_ratio, q, scale, zero, zero8, nullptr,
+                          (hipStream_t)stream)) {
+        SRQ_LAUNCH_CHECK(name);
+        return SRQ_OK;
+    }
+    srq_set_error("%s: no fused form for n=%lld, K=%lld", name, (long long)n, (long long)K);
+    return SRQ_EUNSUPPORTED;
+}
+
 extern "C" int srq_had_sign_asym_quant(const void *x, int64_t rows, int64_t n, int64_t K,
                                        const void *hadK, const int8_t *sign, float clip_ratio,
                                        void *q, void *scale, void *zero, void *stream) {
-    int rc = check_rotation("had_sign_asym_quant", x, rows, n, K, hadK);
-    if (rc) return rc;
-    if (rows == 0) return SRQ_OK;
-    SRQ_CHECK_ARG(q && scale && zero, "had_sign_asym_quant: null output");
-    SRQ_CHECK_ARG(srq_aligned(x, 16) && srq_aligned(q, 16),
-                  "had_sign_asym_quant: x and q must be 16-byte aligned");
-    if (srq_had512_mfma(x, rows, n, K, hadK, sign, clip_ratio, q, scale, nullptr,
-                        (hipStream_t)stream, nullptr, 0, nullptr, 0, zero) ||
-        srq_had_kron_mfma(x, rows, n, K, hadK, sign, clip_ratio, q, scale, zero, nullptr,
-                          (hipStream_t)stream)) {
-        SRQ_LAUNCH_CHECK("had_sign_asym_quant");
-        return SRQ_OK;
-    }
-    srq_set_error("had_sign_asym_quant: no fused form for n=%lld, K=%lld", (long long)n,
-                  (long long)K);
-    return SRQ_EUNSUPPORTED;
+    return had_sign_asym("had_sign_asym_quant", x, rows, n, K, hadK, sign, clip_ratio, q, scale,
+                         zero, nullptr, stream);
+}
+
+extern "C" int srq_had_sign_asym_quant_i8(const void *x, int64_t rows, int64_t n, int64_t K,
+                                          const void *hadK, const int8_t *sign, float clip_ratio,
+                                          void *q, void *scale, int8_t *zero, void *stream) {
+    return had_sign_asym("had_sign_asym_quant_i8", x, rows, n, K, hadK, sign, clip_ratio, q,
+                         scale, nullptr, zero, stream);
 }

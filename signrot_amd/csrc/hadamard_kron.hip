@@ -77,7 +77,8 @@ struct KronArgs {
     float clip;
     uint8_t *q;           // MODE 1, 2: packed codes, rows of n / 2 bytes
     f16 *qscale;          // MODE 1, 2: [rows]
-    f16 *qzero;           // MODE 2: [rows]
+    f16 *qzero;           // MODE 2: [rows] or null
+    int8_t *qzero8;       // MODE 2: the same as int8 or null
     f16 *out;             // MODE 0: rows of n
 };
 
@@ -370,7 +371,8 @@ __global__ __launch_bounds__(MAXT) void had_kron_kernel(KronArgs a) {
                 asym_row_params(rmin, rmax, a.clip, sh, zh);
                 if (threadIdx.x == 0) {
                     a.qscale[row] = sh;
-                    a.qzero[row] = zh;
+                    if (a.qzero) a.qzero[row] = zh;
+                    if (a.qzero8) a.qzero8[row] = zero_i8(zh);
                 }
                 const float sf = (float)sh;
                 const int zi = h2i_rn((float)zh);
@@ -416,11 +418,11 @@ __global__ __launch_bounds__(MAXT) void had_kron_kernel(KronArgs a) {
 }  // namespace
 
 // Launches the kernel above for n = K * m (rotation into `out`; with q, the
-// symmetric quantizer; with q and qzero, the asymmetric one).  Returns 1 if
+// symmetric quantizer; with q and a zero-point output, the asymmetric one).  Returns 1 if
 // it launched, 0 if the size or an alignment is not covered.
 int srq_had_kron_mfma(const void *x, int64_t rows, int64_t n, int64_t K, const void *hadK,
                       const int8_t *sign, float clip, void *q, void *qscale, void *qzero,
-                      void *out, hipStream_t st) {
+                      int8_t *qzero8, void *out, hipStream_t st) {
     if (K < 12 || K > 176 || K % 4 || n % K) return 0;
     // sizes that the LDS kernel refuses (two fp32 rows beyond 160 KiB) stay
     // refused
@@ -440,6 +442,7 @@ int srq_had_kron_mfma(const void *x, int64_t rows, int64_t n, int64_t K, const v
     a.q = (uint8_t *)q;
     a.qscale = (f16 *)qscale;
     a.qzero = (f16 *)qzero;
+    a.qzero8 = qzero8;
     a.out = (f16 *)out;
     bool done = false;
     auto go = [&](auto ks, auto ka, auto p, auto qq, auto maxt, int wi) {
@@ -449,7 +452,7 @@ int srq_had_kron_mfma(const void *x, int64_t rows, int64_t n, int64_t K, const v
         // persistent blocks: enough for the resident ones of 256 CUs
         const int per_cu = std::max<int>(1, 1024 / (int)block.x);
         const dim3 grid((unsigned)std::min<int64_t>(rows, 256 * per_cu));
-        if (q && qzero) had_kron_kernel<KS, KA, P, Q, 2, MT><<<grid, block, 0, st>>>(a);
+        if (q && (qzero || qzero8)) had_kron_kernel<KS, KA, P, Q, 2, MT><<<grid, block, 0, st>>>(a);
         else if (q) had_kron_kernel<KS, KA, P, Q, 1, MT><<<grid, block, 0, st>>>(a);
         else had_kron_kernel<KS, KA, P, Q, 0, MT><<<grid, block, 0, st>>>(a);
         done = true;

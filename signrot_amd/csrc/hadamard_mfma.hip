@@ -88,7 +88,8 @@ struct MfmaRotArgs {
     float clip;
     uint8_t *q;           // quant mode: packed codes, rows of n/2 bytes
     f16 *qscale;          // quant mode: [rows]
-    f16 *qzero;           // asymmetric quant mode: zero points [rows]
+    f16 *qzero;           // asymmetric quant mode: zero points [rows] or null
+    int8_t *qzero8;       // asymmetric quant mode: the same as int8 or null
     f16 *out;             // rotation mode: fp16 rows of n
     const f16 *up;        // SwiGLU input: x is the gate, this the up projection
     int64_t ld;           // row stride of x (and up), elements
@@ -270,7 +271,7 @@ SRQ_DEV void quant_store_asym(const u32 (&w)[4][8], float rcp, v2h lo, v2h hi, v
 // P: 512-chunks per Hadamard chunk (1: H_512, 2: H_1024; one workgroup per
 // CU, which holds twice the row in registers).
 template <int NT, int MODE, bool SW, int P>
-__global__ __launch_bounds__(256, (SW || P == 2 || MODE == 2) ? 1 : 2) void had512_mfma_kernel(
+__global__ __launch_bounds__(256, (SW || P == 2) ? 1 : 2) void had512_mfma_kernel(
     MfmaRotArgs a) {
     // The staged rows, double-buffered (row r of the block's sequence in
     // rowbuf[r & 1]): 128-element segment (chunk c, quarter i1) at
@@ -580,7 +581,8 @@ __global__ __launch_bounds__(256, (SW || P == 2 || MODE == 2) ? 1 : 2) void had5
             asym_row_params(vmin, vmax, a.clip, sh, zh);
             if (threadIdx.x == 0) {
                 a.qscale[r] = sh;
-                a.qzero[r] = zh;
+                if (a.qzero) a.qzero[r] = zh;
+                if (a.qzero8) a.qzero8[r] = zero_i8(zh);
             }
             const float sf = (float)sh;
             const int zi = h2i_rn((float)zh);
@@ -867,7 +869,8 @@ __global__ __launch_bounds__(256, (SW || P == 2 || MODE == 2) ? 1 : 2) void had5
 int srq_had512_mfma(const void *x, int64_t rows, int64_t n, int64_t K, const void *hadK,
                     const int8_t *sign, float clip, void *q, void *qscale, void *out,
                     hipStream_t st, const void *up, int64_t ld, const int32_t *sign_row,
-                    int64_t n_sign_rows, void *qzero, int bf6) {
+                    int64_t n_sign_rows, void *qzero, int bf6, int8_t *qzero8) {
+    const bool asym = qzero || qzero8;
     // K % 4 == 0: the row fetch moves 4 chunks per instruction and the hadK
     // loads take runs of 2 or 4 table entries (every Hadamard order above 2
     // is a multiple of 4)
@@ -879,8 +882,8 @@ int srq_had512_mfma(const void *x, int64_t rows, int64_t n, int64_t K, const voi
     // the SwiGLU form of H_1024 holds gate and up prefetches of a 2K-chunk
     // row: it fits the register file up to K = 28 (K = 32 would spill)
     if (up && P == 2 && K > 28) return 0;
-    if (qzero && (up || !q)) return 0;  // asymmetric codes: plain rows only
-    if (bf6 && (!q || qzero || n % 128 || !srq_aligned(q, 16))) return 0;
+    if (asym && (up || !q)) return 0;  // asymmetric codes: plain rows only
+    if (bf6 && (!q || asym || n % 128 || !srq_aligned(q, 16))) return 0;
     if (ld < n) ld = n;
     if (rows > 0 && ((rows - 1) * ld + n) * 2 >= (int64_t)kOob) return 0;  // 32-bit offsets
     if (!srq_aligned(x, 16) || (up && !srq_aligned(up, 16)) || ld % 8) return 0;
@@ -902,11 +905,13 @@ int srq_had512_mfma(const void *x, int64_t rows, int64_t n, int64_t K, const voi
     a.sign_row = sign_row;
     a.n_sign_rows = n_sign_rows;
     a.qzero = (f16 *)qzero;
+    a.qzero8 = qzero8;
     a.bf6 = bf6;
-    // persistent blocks of 4 waves, up to 2 per CU (256 CUs; 1 with the
-    // SwiGLU input, H_1024 chunks or the asymmetric quantizer), one row each
-    // at a time
-    const int64_t cap = (up || P == 2 || qzero) ? 256 : 256 * 2;
+    // persistent blocks of 4 waves, up to 2 per CU (256 CUs; the asymmetric
+    // quantizer at one block per CU took 19.5 us at 1000 rows of 14336, 15.4
+    // with two; 1 with the
+    // SwiGLU input or H_1024 chunks), one row each at a time
+    const int64_t cap = (up || P == 2) ? 256 : 256 * 2;
     const int64_t blocks = rows < cap ? rows : cap;
     const dim3 grid((unsigned)blocks), block(256);
     auto go = [&](auto ntc, auto modec, auto swc, auto pc) {
@@ -950,7 +955,7 @@ int srq_had512_mfma(const void *x, int64_t rows, int64_t n, int64_t K, const voi
             if (K <= 16) go(I4{}, M1{}, S1{}, P2{});
             else go(I7{}, M1{}, S1{}, P2{});
         }
-    } else if (q && qzero) {
+    } else if (asym) {
         mode(M2{});
     } else if (q) {
         mode(M1{});

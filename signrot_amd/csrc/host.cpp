@@ -159,25 +159,29 @@ PyObject *had_sign_quant(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
     });
 }
 
-// had_sign_asym_quant(x, hadK, K, sign, clip_ratio) -> (q, scale, zero)
+// had_sign_asym_quant(x, hadK, K, sign, clip_ratio, int8_zero) -> (q, scale, zero)
 PyObject *had_sign_asym_quant(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
-    return guarded(n_args, 5, [&]() -> PyObject * {
+    return guarded(n_args, 6, [&]() -> PyObject * {
         int64_t rows, n;
         const at::Tensor &x = rows_of(a[0], rows, n);
         const at::Device dev = x.device();
         const int64_t K = as_int(a[2]);
         void *h = had_table(a[1], K, false, dev), *s = opt_ptr(a[3], kI8, n, dev);
         const float clip = as_float(a[4]);
+        const bool i8 = as_bool(a[5]);
         at::Tensor q, sc, z;
         int rc;
         {
             NoGil nogil;
             q = alloc(with_last(x, n / 2), kU8, dev);
             sc = alloc(with_last(x, 1), kF16, dev);
-            z = alloc(with_last(x, 1), kF16, dev);
-            rc = srq_had_sign_asym_quant(x.data_ptr(), rows, n, K, h, (const int8_t *)s, clip,
-                                         q.data_ptr(), sc.data_ptr(), z.data_ptr(),
-                                         stream_of(dev));
+            z = alloc(with_last(x, 1), i8 ? kI8 : kF16, dev);
+            rc = i8 ? srq_had_sign_asym_quant_i8(x.data_ptr(), rows, n, K, h, (const int8_t *)s,
+                                                 clip, q.data_ptr(), sc.data_ptr(),
+                                                 (int8_t *)z.data_ptr(), stream_of(dev))
+                    : srq_had_sign_asym_quant(x.data_ptr(), rows, n, K, h, (const int8_t *)s,
+                                              clip, q.data_ptr(), sc.data_ptr(), z.data_ptr(),
+                                              stream_of(dev));
         }
         if (rc) throw Bad();
         return wrap({q, sc, z});

@@ -124,13 +124,13 @@ def w4a4_linear_asym(A, a_scale, a_zero, B, b_scale, b_sum, bias=None):
     return out.view(*A_shape_excl_last, B.shape[0])
 
 
-def asym_quant_dynamic(x, clip_ratio=1.0):
+def asym_quant_dynamic(x, clip_ratio=1.0, int8_zero=False):
     """Fused per-row amin/amax + scale/zero + asymmetric uint4 quantize/pack
     (kernel.py:113-120): (q, scale, zero), scale and zero shaped
-    (*x.shape[:-1], 1)."""
+    (*x.shape[:-1], 1); int8_zero: zero as int8."""
     assert x.dtype == torch.float16
     x, shape_excl_last = flatten_last_dim_and_return_shape(x.contiguous())
-    q, scale, zero = _CUDA.asym_quant_dynamic(x, clip_ratio)
+    q, scale, zero = _CUDA.asym_quant_dynamic(x, clip_ratio, int8_zero)
     return (q.view(*shape_excl_last, -1), scale.view(*shape_excl_last, 1),
             zero.view(*shape_excl_last, 1))
 
@@ -259,11 +259,11 @@ def sym_quant_dynamic_moe(x, sign, expert_ids, clip_ratio=1.0):
     return _CUDA.sym_quant_dynamic_moe(x.contiguous(), sign, expert_ids, clip_ratio)
 
 
-def asym_quant_dynamic_moe(x, sign, expert_ids, clip_ratio=1.0):
+def asym_quant_dynamic_moe(x, sign, expert_ids, clip_ratio=1.0, int8_zero=False):
     """asym_quant_dynamic variant of sym_quant_dynamic_moe -> (q, scale,
     zero) (kernel.py:131-134)."""
     assert x.dtype == torch.float16
-    return _CUDA.asym_quant_dynamic_moe(x.contiguous(), sign, expert_ids, clip_ratio)
+    return _CUDA.asym_quant_dynamic_moe(x.contiguous(), sign, expert_ids, clip_ratio, int8_zero)
 
 
 def sym_dequant_moe(q, scale_row, w_scales, expert_ids, zero_row=None, w_sum=None):

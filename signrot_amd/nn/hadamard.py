@@ -123,9 +123,9 @@ class HadamardQuantizer(torch.nn.Module):
         if isinstance(quantizer, AsymQuantizer):
             if h.fp32_had:
                 return quantizer(h(x))
-            q, s, z = _CUDA.had_sign_asym_quant(x.contiguous(), h._hadk(x.device), h.rem_dim,
-                                                h._sign(), quantizer.clip_ratio)
-            return kernel.PackedQuantizedTensor(q, s, z.to(torch.int8))
+            return kernel.PackedQuantizedTensor(
+                *_CUDA.had_sign_asym_quant(x.contiguous(), h._hadk(x.device), h.rem_dim,
+                                           h._sign(), quantizer.clip_ratio, True))
         q, s = kernel.had_sign_quant(x, h._hadk(x.device), h.rem_dim, h._sign(),
                                      quantizer.clip_ratio, h.fp32_had)
         return kernel.PackedQuantizedTensor(q, s)

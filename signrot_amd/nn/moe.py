@@ -131,8 +131,7 @@ class SignRotMoEBlock(torch.nn.Module):
 
     def _quant(self, x) -> _Codes:
         if self.asym:
-            q, s, z = kernel.asym_quant_dynamic(x, self.clip_ratio)
-            return _Codes(q, s, z.to(torch.int8))
+            return _Codes(*kernel.asym_quant_dynamic(x, self.clip_ratio, int8_zero=True))
         q, s = kernel.sym_quant_dynamic(x, self.clip_ratio)
         return _Codes(q, s, None)
 
@@ -140,8 +139,8 @@ class SignRotMoEBlock(torch.nn.Module):
         """Quantizer of the down-proj input with row r flipped by
         sign_down[expert[r]] (fused into the quantizer)."""
         if self.asym:
-            q, s, z = kernel.asym_quant_dynamic_moe(h, self.sign_down, expert, self.clip_ratio)
-            return _Codes(q, s, z.to(torch.int8))
+            return _Codes(*kernel.asym_quant_dynamic_moe(h, self.sign_down, expert,
+                                                         self.clip_ratio, int8_zero=True))
         q, s = kernel.sym_quant_dynamic_moe(h, self.sign_down, expert, self.clip_ratio)
         return _Codes(q, s, None)
 

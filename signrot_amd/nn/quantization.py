@@ -68,8 +68,8 @@ class AsymQuantizer(QuantizerBase):
         self.maxq = get_minq_maxq(bits, sym=False)[1]
 
     def forward(self, x: torch.Tensor) -> kernel.PackedQuantizedTensor:
-        quantized_x, scales_x, zeros_x = kernel.asym_quant_dynamic(x, self.clip_ratio)
-        return kernel.PackedQuantizedTensor(quantized_x, scales_x, zeros_x.to(torch.int8))
+        return kernel.PackedQuantizedTensor(
+            *kernel.asym_quant_dynamic(x, self.clip_ratio, int8_zero=True))
 
     def forward_reference(self, x: torch.Tensor) -> kernel.PackedQuantizedTensor:
         """Unfused composition (quantization.py:69-79): torch min/max/div/round
