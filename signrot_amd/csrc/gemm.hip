@@ -243,12 +243,14 @@ SRQ_DEV int frag_row(int v, int lane) {
     else return 4 * (lane >> 4) + v;
 }
 
-template <int BS, int FM, int FN, bool CHECK, typename AccT>
+// UA: unsigned A (the accumulator is 16 sum, not 256 sum), e.zr may be given.
+template <int BS, int FM, int FN, bool CHECK, bool UA, typename AccT>
 SRQ_DEV void store_block_lds_impl(const Epi &e, int64_t M, int64_t N, int64_t mb, int64_t nb,
                                   const AccT (&acc)[FM][FN], int lane, f16 *tile) {
     constexpr int NV = BS * BS / 64;  // accumulator elements per lane per block
     constexpr int W = BS * FN;        // tile row stride (halves)
     float sbv[FN], bv[FN];
+    u32 wsv[FN];  // asymmetric activations: the columns' weight sums
     int64_t gnv[FN];
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
@@ -256,15 +258,19 @@ SRQ_DEV void store_block_lds_impl(const Epi &e, int64_t M, int64_t N, int64_t mb
         const bool on = !CHECK || gnv[j] < N;
         sbv[j] = on ? (float)e.sb[gnv[j]] : 0.f;
         bv[j] = on && e.bias ? (float)e.bias[gnv[j]] : 0.f;
+        if constexpr (UA) wsv[j] = on && e.zr ? (u32)e.ws[gnv[j]] : 0u;
     }
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
-        // the block's row scales first, all loads in flight together
+        // the block's row scales (and zero points) first, all loads in flight
+        // together
         float sav[NV];
+        int zv[NV];
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
             const int64_t gm = mb + i * BS + frag_row<BS>(v, lane);
             sav[v] = !CHECK || gm < M ? (float)e.sa[gm] : 0.f;
+            if constexpr (UA) zv[v] = e.zr && (!CHECK || gm < M) ? (int)e.zr[gm] : 0;
         }
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
@@ -272,11 +278,8 @@ SRQ_DEV void store_block_lds_impl(const Epi &e, int64_t M, int64_t N, int64_t mb
             const int64_t gm = mb + lr;
 #pragma unroll
             for (int j = 0; j < FN; ++j) {
-                int val = acc[i][j][v] >> (e.ua ? 4 : 8);
-                if (e.zr) {  // (uniform) asymmetric activations
-                    const bool on = !CHECK || (gm < M && gnv[j] < N);
-                    val = on ? epi_val(e, acc[i][j][v], gm, gnv[j]) : 0;
-                }
+                int val = acc[i][j][v] >> (UA ? 4 : 8);
+                if constexpr (UA) val = (int)((u32)val - (u32)zv[v] * wsv[j]);  // epi_val
                 f16 o = f16_rn((float)val * sav[v] * sbv[j]);
                 if (e.bias) o = f16_rn((float)o + bv[j]);
                 tile[lr * W + j * BS + (lane & (BS - 1))] = o;
@@ -350,13 +353,13 @@ SRQ_DEV void store_block_lds_impl(const Epi &e, int64_t M, int64_t N, int64_t mb
 // divergent branches: 20 of the M = 2048 GEMM's 108 us).  Same arithmetic
 // as store_one.  The caller's LDS `tile` must be free of other readers and
 // of in-flight DMA.
-template <int BS, int FM, int FN, typename AccT>
+template <int BS, int FM, int FN, bool UA, typename AccT>
 SRQ_DEV void store_block_lds(const Epi &e, int64_t M, int64_t N, int64_t mb, int64_t nb,
                              const AccT (&acc)[FM][FN], int lane, f16 *tile) {
     if (mb + BS * FM <= M && nb + BS * FN <= N)
-        store_block_lds_impl<BS, FM, FN, false>(e, M, N, mb, nb, acc, lane, tile);
+        store_block_lds_impl<BS, FM, FN, false, UA>(e, M, N, mb, nb, acc, lane, tile);
     else
-        store_block_lds_impl<BS, FM, FN, true>(e, M, N, mb, nb, acc, lane, tile);
+        store_block_lds_impl<BS, FM, FN, true, UA>(e, M, N, mb, nb, acc, lane, tile);
 }
 
 // fp16 epilogue through an int32 LDS tile, for kernels with little register
@@ -366,7 +369,7 @@ SRQ_DEV void store_block_lds(const Epi &e, int64_t M, int64_t N, int64_t mb, int
 // (column scales loaded once per lane, one row scale per row) and stores
 // them as 16 bytes.  Same arithmetic as store_one; `tile` must be free of
 // other readers and of in-flight DMA, 4 BS FN BS FM bytes.
-template <int BS, int FM, int FN, typename AccT>
+template <int BS, int FM, int FN, bool UA, typename AccT>
 SRQ_DEV void store_block_lds32(const Epi &e, int64_t M, int64_t N, int64_t mb, int64_t nb,
                                const AccT (&acc)[FM][FN], int lane, int32_t *tile) {
     constexpr int NV = BS * BS / 64;
@@ -391,6 +394,12 @@ SRQ_DEV void store_block_lds32(const Epi &e, int64_t M, int64_t N, int64_t mb, i
     for (int k = 0; k < 8; ++k) sbv[k] = gn0 + k < N ? (float)e.sb[gn0 + k] : 0.f;
     const bool vec = full_n && N % 8 == 0 && ((uintptr_t)e.out % 16 == 0) &&
                      (!e.res || (uintptr_t)e.res % 16 == 0);
+    // asymmetric activations: the columns' weight sums once per lane
+    u32 wsv[8] = {};
+    if (UA && e.zr) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) wsv[k] = gn0 + k < N ? (u32)e.ws[gn0 + k] : 0u;
+    }
     for (int r0 = 0; r0 < BS * FM; r0 += RPI) {
         const int lr = r0 + lane / LPR;
         const int64_t gm = mb + lr;
@@ -398,11 +407,13 @@ SRQ_DEV void store_block_lds32(const Epi &e, int64_t M, int64_t N, int64_t mb, i
         const v4i a0 = *reinterpret_cast<const v4i *>(tile + lr * WS + c8);
         const v4i a1 = *reinterpret_cast<const v4i *>(tile + lr * WS + c8 + 4);
         const float sa = (float)e.sa[gm];
+        const u32 z = UA && e.zr ? (u32)(int)e.zr[gm] : 0u;
         v8h o;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const int a = k < 4 ? a0[k] : a1[k - 4];
-            const int val = epi_val(e, a, gm, gn0 + k < N ? gn0 + k : gn0);
+            int val = a >> (UA ? 4 : 8);
+            if constexpr (UA) val = (int)((u32)val - z * wsv[k]);  // epi_val
             f16 x = f16_rn((float)val * sa * sbv[k]);
             // bias read per row pass (cached), not held in 8 more registers
             if (e.bias && gn0 + k < N) x = f16_rn((float)x + (float)e.bias[gn0 + k]);
@@ -715,7 +726,7 @@ __global__ __launch_bounds__(64 * (WGM * WGN + NPROD), 1) void gemm_big_kernel(
         uint8_t *fr0 = smem + (steps % 3) * kStage, *fr1 = smem + ((steps + 1) % 3) * kStage;
         const int per0 = kStage / kTile;
         uint8_t *t = wave < per0 ? fr0 + wave * kTile : fr1 + (wave - per0) * kTile;
-        store_block_lds<32, FM, FN>(e, M, N, m0 + wm * (FM * 32), n0 + wn * (FN * 32), acc, lane,
+        store_block_lds<32, FM, FN, UA>(e, M, N, m0 + wm * (FM * 32), n0 + wn * (FN * 32), acc, lane,
                                   reinterpret_cast<f16 *>(t));
     }
 }
@@ -840,7 +851,7 @@ __global__ __launch_bounds__(512, 1) void gemm_sq_kernel(const uint8_t *__restri
         static_assert(kWaves * kTile <= NSTG * kStage, "epilogue tiles");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        store_block_lds<32, FM, FN>(e, M, N, m0 + wm * (FM * 32), n0 + wn * (FN * 32), acc, lane,
+        store_block_lds<32, FM, FN, UA>(e, M, N, m0 + wm * (FM * 32), n0 + wn * (FN * 32), acc, lane,
                                     reinterpret_cast<f16 *>(smem + wave * kTile));
     }
 }
@@ -996,7 +1007,7 @@ __global__ __launch_bounds__(64 * (4 + NPROD), 1) void gemm_ring_kernel(const ui
         constexpr int kTile = WM * WN * 2;
         static_assert(NSTG >= 2 && 4 * kTile <= kStage, "epilogue tiles");
         uint8_t *fr = smem + (steps % NSTG) * kStage;
-        store_block_lds<16, FM, FN>(e, M, N, m0 + wm * WM, n0 + wn * WN, acc, lane,
+        store_block_lds<16, FM, FN, UA>(e, M, N, m0 + wm * WM, n0 + wn * WN, acc, lane,
                                     reinterpret_cast<f16 *>(fr + wave * kTile));
     }
 }
@@ -1852,7 +1863,7 @@ __global__ __launch_bounds__(64 * (4 + NPROD), 1) void gemm_grouped_kernel(Group
                     e, pr.m, pr.n, m0 + wm * (FM * 32), n0 + wn * (FN * 32), acc, lane,
                     reinterpret_cast<int32_t *>(epi_lds + wave * kEpiTile));
             else
-                store_block_lds32<32, FM, FN>(e, pr.m, pr.n, m0 + wm * (FM * 32),
+                store_block_lds32<32, FM, FN, UA>(e, pr.m, pr.n, m0 + wm * (FM * 32),
                                               n0 + wn * (FN * 32), acc, lane,
                                               reinterpret_cast<int32_t *>(epi_lds + wave * kEpiTile));
             continue;
@@ -2052,7 +2063,7 @@ __global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
                 store_block_lds32_swiglu<32, 1, 1>(e, pr.m, pr.n, m0 + 32 * i, n0 + wave * 32, one,
                                                    lane, tile);
             else
-                store_block_lds32<32, 1, 1>(e, pr.m, pr.n, m0 + 32 * i, n0 + wave * 32, one, lane,
+                store_block_lds32<32, 1, 1, UA>(e, pr.m, pr.n, m0 + 32 * i, n0 + wave * 32, one, lane,
                                             tile);
         }
     }
