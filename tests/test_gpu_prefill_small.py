@@ -1,0 +1,51 @@
+"""Prefill attention of short causal prompts (32-row blocks of 4 heads, and the
+form whose wave sets share the key tiles) against float32 attention: lengths
+at the edges of tiles, steps and of the rule that picks the form, groups of 4
+and 8, left padding down to one live token, strided inputs."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+D = 128
+
+
+def _ref(q, k, v, mask):
+    B, T, Hq, _ = q.shape
+    g = Hq // k.shape[2]
+    out = torch.zeros(B, T, Hq, D, device="cuda")
+    causal = torch.ones(T, T, dtype=torch.bool, device="cuda").tril()
+    for b in range(B):
+        ok = causal if mask is None else causal & (mask[b] != 0)[None, :]
+        for h in range(Hq):
+            s = q[b, :, h].float() @ k[b, :, h // g].float().T * D ** -0.5
+            p = torch.softmax(s.masked_fill(~ok, -1e30), -1)
+            o = p @ v[b, :, h // g].float()
+            if mask is not None:
+                o = o * (mask[b] != 0)[:, None]
+            out[b, :, h] = o
+    return out
+
+
+# (8, 8) etc: query heads, KV heads.  32-row blocks, 64-key tiles, 128-key steps
+@pytest.mark.parametrize("Hq,Hkv", [(8, 2), (16, 2), (32, 8), (4, 1)])
+@pytest.mark.parametrize("B,T", [(1, 1), (1, 31), (2, 64), (1, 65), (1, 256), (1, 257), (2, 300),
+                                 (1, 384), (1, 449), (3, 400), (1, 700), (1, 1025)])
+@pytest.mark.parametrize("padded", [False, True])
+def test_short_prompts(Hq, Hkv, B, T, padded):
+    from signrot_amd import _CUDA as C
+    gen = torch.Generator("cuda").manual_seed(T + Hq)
+    heads = torch.randn(B, T, Hq + 2 * Hkv, D, device="cuda", generator=gen).half()
+    q, k, v = heads.split((Hq, Hkv, Hkv), dim=2)   # strided views
+    q = q * 2
+    mask = None
+    if padded:
+        pad = torch.tensor([(7 * b + 1) * T // 9 for b in range(B)], device="cuda")
+        pad[0] = T - 1                             # one live token
+        mask = (torch.arange(T, device="cuda")[None] >= pad[:, None]).int()
+    out = C.prefill_attention(q, k, v, mask).float()
+    want = _ref(q, k, v, mask)
+    # fp16 probabilities and outputs: 2^-11 relative each
+    assert torch.allclose(out, want, rtol=4e-3, atol=4e-3)
+    if mask is not None:
+        assert torch.all(out[mask == 0] == 0)
