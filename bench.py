@@ -610,7 +610,8 @@ def gemm_kernel_name(M, N, K=None, split=False):
         return "gemm_rows_kernel split-K form + splitk_reduce_kernel (srq_w4a4_linear_ws)"
     if M <= 64:
         return "gemm_skinny_kernel (srq_w4a4_linear)"
-    if M >= 1024 and cdiv(M, 256) * cdiv(N, 256) >= 256:
+    sq, big = cdiv(M, 256) * cdiv(N, 256), cdiv(M, 256) * cdiv(N, 128)
+    if M >= 1024 and 7 * cdiv(sq, 256) <= 4 * cdiv(big, 256):
         return "gemm_sq_kernel (srq_w4a4_linear, 256 x 256 tiles)"
     if split:
         return "gemm_grouped_kernel split-K form + splitk_reduce_kernel (srq_w4a4_linear_ws)"

@@ -2307,6 +2307,19 @@ void splitk_reduce(const void *ws, int S, int64_t M, int64_t N, const Epi &e, hi
     }
 }
 
+// Square or 256 x 128 tiles for a large product: by the rounds of the 256 CUs
+// that each takes, a round of square tiles being about 1.75 of the others
+// (twice the work, less data movement); square where they tie.  us, K = 4096,
+// weights from memory: M = 2048, N = 6144 (192 against 384 tiles) square 53,
+// 256 x 128 58; M = 1500, N = 6144 55, 61; M = 1024, N = 14336 (224, 448) 57, 63;
+// M = 1200, N = 28672 (560, 1120) 163, 159; M = 2048, N = 28672 (896, 1792; tie)
+// 228, 241; M = 2048, N = 4096 (128, 256) 51, 35.
+bool use_square_tiles(int64_t M, int64_t N) {
+    const int64_t sq = srq_cdiv(M, kSqBM) * srq_cdiv(N, kSqBN);
+    const int64_t big = srq_cdiv(M, kBigBM) * srq_cdiv(N, kBigBN);
+    return 7 * srq_cdiv(sq, 256) <= 4 * srq_cdiv(big, 256);
+}
+
 // One dense problem with e's fp16 epilogue.
 GroupedArgs dense_args(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K,
                        const Epi &e) {
@@ -2360,8 +2373,7 @@ void launch_gemm(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64
     } else if (M <= 64 && !e.swiglu) {
         gemm_skinny_kernel<4, 8, 2, UA><<<dim3((unsigned)srq_cdiv(N, 16), 1), dim3(512), 0, st>>>(
             a, b, M, N, K, e);
-    } else if (M >= 1024 && srq_cdiv(M, kSqBM) * srq_cdiv(N, kSqBN) >= 256) {
-        // enough 256 x 256 tiles to cover the 256 CUs
+    } else if (M >= 1024 && use_square_tiles(M, N)) {
         const int64_t tiles = srq_cdiv(M, kSqBM) * srq_cdiv(N, kSqBN);
         gemm_sq_kernel<128, 2, UA><<<dim3((unsigned)tiles), dim3(512), 0, st>>>(a, b, M, N, K, e);
     } else if (sk.S && sk.big && !e.swiglu && ws_bytes >= (int64_t)sk.S * M * N * 4) {
