@@ -125,7 +125,22 @@ struct QkvArgs {
     f16 *q_out;          // [B, hq, D]
 };
 
-SRQ_DEV float xor_lane(float v, int m) { return __shfl_xor(v, m, 64); }
+// The value of lane l ^ M within each 16-lane row, by DPP: a vector move, where
+// __shfl_xor is a trip through the LDS crossbar (48 of them a row here).
+template <int CTRL>
+SRQ_DEV float dpp_mov(float x) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, true));
+}
+
+template <int M>
+SRQ_DEV float xor_lane(float v) {
+    static_assert(M == 1 || M == 2 || M == 4 || M == 8, "within a row of 16 lanes");
+    if constexpr (M == 1) return dpp_mov<0xB1>(v);           // quad_perm [1, 0, 3, 2]
+    if constexpr (M == 2) return dpp_mov<0x4E>(v);           // quad_perm [2, 3, 0, 1]
+    if constexpr (M == 4) return dpp_mov<0x1B>(dpp_mov<0x141>(v));  // l ^ 7, then l ^ 3
+    return dpp_mov<0x128>(v);                                // row_ror:8
+}
 
 // The per-row arithmetic, shared by qkv_post_kernel and the fused form of
 // decode_kernel so that both give the same bits.  Lane l (0..15) of a
@@ -138,7 +153,7 @@ SRQ_DEV void qkv_row_rope(float (&v)[8], int kind, int l, const f16 *cs, const f
     float y[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        const float o = xor_lane(v[e], 8);
+        const float o = xor_lane<8>(v[e]);
         const int i = 8 * l + e;
         const f16 c = cs[ct * D + i], s = sn[ct * D + i];
         const f16 xe = (f16)v[e], xo = (f16)o;  // exact: both came from fp16
@@ -150,19 +165,24 @@ SRQ_DEV void qkv_row_rope(float (&v)[8], int kind, int l, const f16 *cs, const f
     }
 }
 
+template <int M>
+SRQ_DEV void fwht_lanes(float (&w)[8], int l) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float o = xor_lane<M>(w[e]);
+        w[e] = (l & M) ? o - w[e] : w[e] + o;
+    }
+}
+
 SRQ_DEV void qkv_row_had(float (&v)[8], int kind, int l, float had_scale) {
     float w[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) w[e] = v[e];
     fwht_regs<8>(w);
-#pragma unroll
-    for (int m = 1; m < 16; m <<= 1) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float o = xor_lane(w[e], m);
-            w[e] = (l & m) ? o - w[e] : w[e] + o;
-        }
-    }
+    fwht_lanes<1>(w, l);
+    fwht_lanes<2>(w, l);
+    fwht_lanes<4>(w, l);
+    fwht_lanes<8>(w, l);
     if (kind != 2) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = (float)f16_rn(w[e] * had_scale);
@@ -177,6 +197,12 @@ SRQ_DEV void qkv_row_transform(float (&v)[8], int kind, int l, const f16 *cs, co
 
 // KV int4 quantizer of a transformed row: the row max / min over the 16
 // lanes, [scale, zero], and this lane's 8 codes as one word.
+template <int M>
+SRQ_DEV void max_min_lanes(float &vmax, float &vmin) {
+    vmax = fmaxf(vmax, xor_lane<M>(vmax));
+    vmin = fminf(vmin, xor_lane<M>(vmin));
+}
+
 SRQ_DEV u32 kv_row_codes(const float (&v)[8], f16 &scale, f16 &zero) {
     float vmax = -INFINITY, vmin = INFINITY;
 #pragma unroll
@@ -184,11 +210,10 @@ SRQ_DEV u32 kv_row_codes(const float (&v)[8], f16 &scale, f16 &zero) {
         vmax = fmaxf(vmax, v[e]);
         vmin = fminf(vmin, v[e]);
     }
-#pragma unroll
-    for (int m = 1; m < 16; m <<= 1) {
-        vmax = fmaxf(vmax, xor_lane(vmax, m));
-        vmin = fminf(vmin, xor_lane(vmin, m));
-    }
+    max_min_lanes<1>(vmax, vmin);
+    max_min_lanes<2>(vmax, vmin);
+    max_min_lanes<4>(vmax, vmin);
+    max_min_lanes<8>(vmax, vmin);
     kv_row_params(vmax, vmin, scale, zero);
     const float fs = (float)scale, fz = (float)zero;
     u32 word = 0;
@@ -254,10 +279,14 @@ __global__ __launch_bounds__(256) void qkv_post_kernel(QkvArgs a, Paged p) {
 // arithmetic as rope_qk, hadamard_transform, kv_quant_pack and init_kv_i4 in
 // turn, one pass over the projection output instead of copies of the q, k
 // and v slices and a pass each.  Sixteen lanes per 128-wide row as above; the
-// rotation and the quantizer run only in waves that hold a k or v row.
-// 8B widths (32 + 2 x 8 heads), T = 2048: the ops it stands
-// for took 17 (slices) + 22 (RoPE) + 13 (FWHT) + 2 x 4.8 (quantizers) + 5.7 us
-// (cache fill).
+// rotation and the quantizer run only in waves that hold a k or v row.  Memory
+// bounds it (every row read, the q and k rows written back), once the rest is
+// out of the way: a block works on one token, so that the divisions and the
+// page lookup are done once a wave and not once a row, and the lanes exchange
+// by DPP.  8B widths (32 + 2 x 8 heads), T = 2048: 13.3 us (3.5 TB/s; 17.5 with
+// a row index and shuffles for each row), 4 x 2048 tokens of 64 + 2 x 8 heads
+// 70.5 (86); the ops it stands for took 17 (slices) + 22 (RoPE) + 13 (FWHT) +
+// 2 x 4.8 (quantizers) + 5.7 us (cache fill).
 struct PrefillQkvArgs {
     f16 *qkv;              // [B, T, hq + 2 hk, D]
     const f16 *cs, *sn;    // [cos_batch, T, D]
@@ -272,38 +301,44 @@ __global__ __launch_bounds__(256) void prefill_qkv_kernel(PrefillQkvArgs a, Page
     constexpr int D = 128;
     const int l = threadIdx.x & 15;
     const int hs = a.hq + 2 * a.hk;
-    const int64_t row = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
-    const bool valid = row < a.B * a.T * hs;
-    const int64_t tok = valid ? row / hs : 0;
-    const int slot = valid ? (int)(row - tok * hs) : 0;
-    const int kind = slot < a.hq ? 0 : (slot < a.hq + a.hk ? 1 : 2);  // q, k, v
-    const int64_t b = tok / a.T, t = tok - b * a.T;
-    v8h x = valid ? *reinterpret_cast<const v8h *>(a.qkv + row * D + 8 * l) : (v8h){};
-    int64_t pos = -1, page = 0;
-    if (valid && kind != 0) {
-        pos = seq_len_of(p, b) - a.T + t;
-        if (pos >= 0) page = p.indices[p.indptr[b] + pos / p.page];
+    const int64_t tok = blockIdx.x;
+    const int64_t b = (uint32_t)blockIdx.x / (uint32_t)a.T, t = tok - b * a.T;
+    const int64_t pos = seq_len_of(p, b) - a.T + t;
+    // slot 0's index in the codes and parameters: the token's page and entry
+    int64_t ri0 = 0;
+    if (pos >= 0) {
+        const int64_t pg = pos / p.page;
+        ri0 = row_index(p, p.indices[p.indptr[b] + pg], 0, 0, pos - pg * p.page);
     }
-    float v[8];
+    const int64_t ct = a.cos_batch == 1 ? t : tok;
+    for (int s0 = 16 * blockIdx.y; s0 < hs; s0 += 16 * gridDim.y) {
+        const int slot = s0 + (threadIdx.x >> 4);
+        const bool valid = slot < hs;
+        const int kind = !valid || slot < a.hq ? 0 : (slot < a.hq + a.hk ? 1 : 2);  // q, k, v
+        f16 *row = a.qkv + (tok * hs + slot) * D + 8 * l;
+        v8h x = valid ? *reinterpret_cast<const v8h *>(row) : (v8h){};
+        float v[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = (float)x[e];
-    if (__builtin_amdgcn_ballot_w64(kind != 2) != 0) {
-        qkv_row_rope(v, kind, l, a.cs, a.sn, a.cos_batch == 1 ? t : tok);
-        if (valid && kind != 2) {
+        for (int e = 0; e < 8; ++e) v[e] = (float)x[e];
+        if (__builtin_amdgcn_ballot_w64(kind != 2) != 0) {
+            qkv_row_rope(v, kind, l, a.cs, a.sn, ct);
+            if (valid && kind != 2) {
 #pragma unroll
-            for (int e = 0; e < 8; ++e) x[e] = (f16)v[e];
-            *reinterpret_cast<v8h *>(a.qkv + row * D + 8 * l) = x;
+                for (int e = 0; e < 8; ++e) x[e] = (f16)v[e];
+                *reinterpret_cast<v8h *>(row) = x;
+            }
+        }
+        if (__builtin_amdgcn_ballot_w64(kind != 0) == 0) continue;  // q rows only
+        if (a.rotate) qkv_row_had(v, kind, l, a.had_scale);
+        f16 scale, zero;
+        const u32 word = kv_row_codes(v, scale, zero);
+        if (kind != 0 && pos >= 0) {
+            // k slots 0 .. hk - 1, then v slots: [kv][head] of the cache in order
+            const int64_t ri = ri0 + (int64_t)(slot - a.hq) * p.page;
+            reinterpret_cast<u32 *>(p.data + ri * (D / 2))[l] = word;
+            if (l == 0) reinterpret_cast<uint32_t *>(p.param)[ri] = pack_param(scale, zero);
         }
     }
-    if (__builtin_amdgcn_ballot_w64(kind != 0) == 0) return;  // q rows only
-    if (a.rotate) qkv_row_had(v, kind, l, a.had_scale);
-    f16 scale, zero;
-    const u32 word = kv_row_codes(v, scale, zero);
-    if (!valid || kind == 0 || pos < 0) return;
-    const int64_t h = slot - a.hq - (kind == 2 ? a.hk : 0);
-    const int64_t ri = row_index(p, page, kind - 1, h, pos % p.page);
-    reinterpret_cast<u32 *>(p.data + ri * (D / 2))[l] = word;
-    if (l == 0) reinterpret_cast<uint32_t *>(p.param)[ri] = pack_param(scale, zero);
 }
 
 // --------------------------------------------------------------- decode
@@ -1409,9 +1444,14 @@ extern "C" int srq_prefill_qkv_cache(void *qkv, const void *cos, const void *sin
     a.rotate = rotate ? 1 : 0;
     Paged p = make_paged(kv_data, kv_param, kv_indptr, kv_indices, last_page_offset, num_layers,
                          layer_idx, n_kv_heads, page_size, head_dim);
-    const int64_t blocks = srq_cdiv(batch * seq_len * (n_q_heads + 2 * n_kv_heads), 16);
-    SRQ_CHECK_ARG(blocks <= 0x7fffffffLL, "%s: too many rows", name);
-    prefill_qkv_kernel<<<dim3((unsigned)blocks), 256, 0, (hipStream_t)stream>>>(a, p);
+    SRQ_CHECK_ARG(batch * seq_len <= 0x7fffffffLL, "%s: too many tokens", name);
+    const int64_t passes = srq_cdiv(n_q_heads + 2 * n_kv_heads, 16);
+    // few tokens: a token's passes over several blocks, to about 2048 of them
+    // (us with 1 / 2 / 3 blocks a token, 48 rows a token: 101 tokens 4.5, 4.1,
+    // 3.8; 1024 8.9, 8.4, 9.5; 2048 13.3, 13.8, 14.2)
+    const int64_t ys = std::min<int64_t>(srq_cdiv(2048, batch * seq_len), passes);
+    prefill_qkv_kernel<<<dim3((unsigned)(batch * seq_len), (unsigned)ys), 256, 0,
+                         (hipStream_t)stream>>>(a, p);
     SRQ_LAUNCH_CHECK(name);
     return SRQ_OK;
 }
