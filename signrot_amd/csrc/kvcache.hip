@@ -897,31 +897,57 @@ __global__ __launch_bounds__(NW * 64, NW == 4 ? 3 : 1) void decode_kernel(Decode
     }
 }
 
-// Merge of the per-chunk (o, m, d) records of one (request, query head) at
-// dim d: o = sum_c o_c 2^(m_c - m) / sum_c d_c 2^(m_c - m), m = max_c m_c
-// (decode.cuh:726-751), fp16.
-SRQ_DEV f16 merge_rec(const float *rec, int chunks, int d) {
-    float mx = -INFINITY;
-    for (int c = 0; c < chunks; ++c) mx = fmaxf(mx, rec[c * (kD + 4) + kD]);
-    float ov = 0.f, dv = 0.f;
-    for (int c = 0; c < chunks; ++c) {
-        const float mc = rec[c * (kD + 4) + kD];
-        const float sc = mc == -INFINITY ? 0.f : exp2f(mc - mx);
-        ov += rec[c * (kD + 4) + d] * sc;
-        dv += rec[c * (kD + 4) + kD + 1] * sc;
-    }
-    return (f16)(dv > 0.f ? ov / dv : 0.f);
-}
-
 // (head, chunk) records one merge_head_had_quant block stages in LDS (64 KiB)
 constexpr int kMergeHhqMaxRecords = 65536 / ((kD + 4) * 4);
 static_assert(kMergeHhqMaxRecords * ((kD + 4) / 4) <= 16 * 256, "record copy: 16 float4 / thread");
 
+// Merge of the per-chunk (o, m, d) records of one (request, query head) at
+// dim d: o = sum_c o_c 2^(m_c - m) / sum_c d_c 2^(m_c - m), m = max_c m_c
+// (decode.cuh:726-751), fp16, the sums in chunk order.  A block per head and
+// a thread per dim.  Latency bounds it (a few KiB a block): the first kMergeO
+// chunks' values and, a chunk per thread, the m_c and d_c are all asked for
+// before anything is waited for, and the weights are made once per block.
+// 8 requests x 64 heads x 8 chunks: the attention with it 20.5 us, 23.9 with a
+// chunk's loads after the other's in each thread.
+constexpr int kMergeO = 16;
+constexpr int kMaxChunks = 1024;
 __global__ __launch_bounds__(128) void merge_kernel(const float *__restrict__ tmp, f16 *__restrict__ o,
                                                     int64_t Hq, int chunks) {
+    __shared__ float ms[kMaxChunks], ds[kMaxChunks];
+    __shared__ float wmax[2];
     const int64_t bh = blockIdx.x;
     const int d = threadIdx.x;
-    o[bh * kD + d] = merge_rec(tmp + bh * chunks * (kD + 4), chunks, d);
+    const float *rec = tmp + bh * chunks * (kD + 4);
+    float ov[kMergeO];
+#pragma unroll
+    for (int c = 0; c < kMergeO; ++c) ov[c] = rec[min(c, chunks - 1) * (kD + 4) + d];
+    float mx = -INFINITY;
+    for (int c = d; c < chunks; c += 128) {
+        const float m = rec[c * (kD + 4) + kD];
+        ds[c] = rec[c * (kD + 4) + kD + 1];
+        ms[c] = m;
+        mx = fmaxf(mx, m);
+    }
+#pragma unroll
+    for (int k = 1; k < 64; k <<= 1) mx = fmaxf(mx, __shfl_xor(mx, k, 64));
+    if ((d & 63) == 0) wmax[d >> 6] = mx;
+    __syncthreads();
+    mx = fmaxf(wmax[0], wmax[1]);
+    for (int c = d; c < chunks; c += 128) ms[c] = ms[c] == -INFINITY ? 0.f : exp2f(ms[c] - mx);
+    __syncthreads();
+    float num = 0.f, den = 0.f;
+#pragma unroll
+    for (int c = 0; c < kMergeO; ++c)
+        if (c < chunks) {
+            num += ov[c] * ms[c];
+            den += ds[c] * ms[c];
+        }
+#pragma unroll 8
+    for (int c = kMergeO; c < chunks; ++c) {
+        num += rec[c * (kD + 4) + d] * ms[c];
+        den += ds[c] * ms[c];
+    }
+    o[bh * kD + d] = (f16)(den > 0.f ? num / den : 0.f);
 }
 
 // ------------------------------------------------- head Hadamard + quant
@@ -972,7 +998,7 @@ __global__ __launch_bounds__(256) void head_had_quant_kernel(const f16 *__restri
             if (i < n4) reinterpret_cast<v4f *>(recs)[i] = t[k];
         }
         __syncthreads();
-        // per head: the chunk weights and the denominator (merge_rec's
+        // per head: the chunk weights and the denominator (merge_kernel's
         // arithmetic and order)
         if (threadIdx.x < H) {
             const int h = threadIdx.x;
