@@ -2076,7 +2076,10 @@ void launch_rows(const GroupedArgs &g, int fmb, int64_t tiles, hipStream_t st) {
     if constexpr (FORM == kFormGeneral || FORM == kFormSwiglu) {
         if (fmb == 1) gemm_rows_kernel<1, UA, FORM, 7><<<grid, block, 0, st>>>(g);
         else if (fmb == 2) gemm_rows_kernel<2, UA, FORM, 6><<<grid, block, 0, st>>>(g);
-        else gemm_rows_kernel<3, UA, FORM, 5><<<grid, block, 0, st>>>(g);
+        else if (FORM == kFormSwiglu || fmb == 3)
+            gemm_rows_kernel<3, UA, FORM, 5><<<grid, block, 0, st>>>(g);
+        else
+            gemm_rows_kernel<5, UA, kFormGeneral, 4><<<grid, block, 0, st>>>(g);
     } else {
         if (fmb <= 2) gemm_rows_kernel<2, UA, FORM, 6><<<grid, block, 0, st>>>(g);
         else if (fmb == 3) gemm_rows_kernel<3, UA, FORM, 5><<<grid, block, 0, st>>>(g);
@@ -2098,9 +2101,15 @@ void launch_rows(const GroupedArgs &g, int fmb, int64_t tiles, hipStream_t st) {
 //   2 blocks         76 / 43   107 / 52    109 / 52    111 / 53    115 / 53    166 / 87
 //   3 blocks                                                       127 / 61    132 / 62
 // 80 rows per expert: 153 / 71 -> 139 / 64 with 3 blocks; 96: 161 / 72
-// against 193 / 98.
-int moe_row_blocks(int64_t rows, int64_t experts, int64_t K) {
+// against 193 / 98.  Forms without the extra rows of the 128-row kernel (asymmetric
+// activations, the gate and up pair) take a second tile for an expert of 129
+// rows: 5 blocks where most experts have 129 to 160.  Pair / asymmetric down:
+//   rows per expert    120         124         128         136         144         150
+//   128-row kernel  188 / 114   212 / 115   243 / 120   266 / 126   277 / 127   276 / 123
+//   5 blocks        194 / 90    198 / 86    196 / 90    201 / 90    201 / 90    226 / 143
+int moe_row_blocks(int64_t rows, int64_t experts, int64_t K, bool extra_rows) {
     if (K < 32) return 0;
+    if (!extra_rows && rows > 122 * experts && rows <= 146 * experts) return 5;
     if (rows <= 20 * experts) return 1;
     if (rows <= 48 * experts) return 2;
     if (rows <= 80 * experts) return 3;
@@ -2109,7 +2118,7 @@ int moe_row_blocks(int64_t rows, int64_t experts, int64_t K) {
 
 template <bool UA, int FORM>
 void launch_moe(const GroupedArgs &g, int64_t rows, hipStream_t st) {
-    const int fmb = moe_row_blocks(rows, g.pair ? g.P / 2 : g.P, g.K);
+    const int fmb = moe_row_blocks(rows, g.pair ? g.P / 2 : g.P, g.K, FORM == kFormSwiglu || g.skip_rem);
     if (fmb) {
         GroupedArgs r = g;
         r.skip_rem = 0;
