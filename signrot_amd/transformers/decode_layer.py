@@ -223,7 +223,8 @@ class W4A4LlamaDecodeLayer(torch.nn.Module):
     def _prefill_fused(self, hidden_states, cache, cos, sin, attention_mask):
         """rmsnorm_quant -> q/k/v GEMM -> prefill_qkv_cache (RoPE in place, K
         Hadamard, KV quantize + cache fill; the op-by-op update when padding
-        has to be left out of the cache) -> prefill attention over the strided
+        has to be left out of the cache, or the cache is an adapter that has
+        only update()) -> prefill attention over the strided
         views -> head_had_quant -> o_proj GEMM + residual -> rmsnorm_quant ->
         gate/up GEMM with the SwiGLU in its epilogue -> had_sign_quant -> down
         GEMM + residual."""
@@ -233,8 +234,9 @@ class W4A4LlamaDecodeLayer(torch.nn.Module):
         n1, n2 = self.input_layernorm, self.post_attention_layernorm
         q1, s1 = _CUDA.rmsnorm_quant(x2, n1.eps, n1.mean_dim)
         qkv = _CUDA.w4a4_linear(q1, s1.view(-1), self.w_qkv, self.s_qkv)
-        if attention_mask is None:
-            q, k, v = cache.update_qkv_prefill(qkv.view(B, T, -1), cos, sin, self.layer_idx, Hq)
+        fill = None if attention_mask is not None else getattr(cache, "update_qkv_prefill", None)
+        if fill is not None:
+            q, k, v = fill(qkv.view(B, T, -1), cos, sin, self.layer_idx, Hq)
         else:
             heads = qkv.view(B, T, Hq + 2 * Hk, D).split((Hq, Hk, Hk), dim=2)
             q, k, v = (t.contiguous() for t in heads)

@@ -76,3 +76,19 @@ def test_fused_prefill_refuses_a_filled_layer():
     with pytest.raises(ValueError):
         layer.prefill(h, cache, cos, sin)
     assert cache.length == 8
+
+
+def test_prefill_through_cache_adapter():
+    """A cache that has only the HF methods takes the prefill too."""
+    from signrot_amd.transformers import HFCacheAdapter, MultiLayerPagedKVCache4Bit
+    T, layer = 33, _layer(1024, 8, 2, 896)
+    h = torch.randn(1, T, 1024, device="cuda").half()
+    cos, sin = _cos_sin(1, T, False)
+    outs = []
+    for wrap in (lambda c: c, HFCacheAdapter):
+        cache = MultiLayerPagedKVCache4Bit(1, 16, T, "cuda", 1, 2, D, group_size=4)
+        cache.pages.zero_()
+        cache.scales.zero_()
+        outs.append((layer.prefill(h, wrap(cache), cos, sin), cache.pages, cache.scales))
+    for a, b in zip(*outs):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
