@@ -553,8 +553,9 @@ def had_sign_asym_quant(x, hadK, K, sign=None, clip_ratio=1.0, int8_zero=False):
     zero = torch.empty((*x.shape[:-1], 1), dtype=torch.int8 if int8_zero else torch.float16,
                        device=x.device)
     if rows:
-        _call("srq_had_sign_asym_quant_i8" if int8_zero else "srq_had_sign_asym_quant", _ptr(x), rows, n, int(K), _ptr(hadK), _ptr(sign),
-              float(clip_ratio), _ptr(q), _ptr(scale), _ptr(zero), _stream(x))
+        _call("srq_had_sign_asym_quant_i8" if int8_zero else "srq_had_sign_asym_quant", _ptr(x),
+              rows, n, int(K), _ptr(hadK), _ptr(sign), float(clip_ratio), _ptr(q), _ptr(scale),
+              _ptr(zero), _stream(x))
     return q, scale, zero
 
 
