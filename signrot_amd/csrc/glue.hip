@@ -14,7 +14,7 @@
 namespace {
 
 // ------------------------------------------------------------------ RMSNorm
-// One row per 64-lane wave (rows < 2048 values: 16-byte loads, the row in
+// One row per 64-lane wave (rows <= 8192 values: 16-byte loads, the row in
 // registers, one wave reduction), 4 rows per block.  QUANT additionally
 // quantizes the normalized fp16 row (per-token symmetric int4, the
 // sym_quant_dynamic arithmetic) while it is still in registers; `out` may
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const f16 *__restrict__ x,
     }
 }
 
-// Block per row for few rows (decode batches) and long rows: the 256 threads of a block
+// Block per row for few rows (decode batches): the 256 threads of a block
 // share one row (VPT vectors of 8 each), so a row's VALU work is spread over
 // four waves instead of one; the sum and the maximum cross the waves through
 // LDS.  The maximum (NaN-skipping fmaxf) and the non-finite flag do not
@@ -216,22 +216,16 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const f16 *__restrict__ g,
 
 }  // namespace
 
-// A block per row (rmsnorm_row_kernel) for rows of 2048 values and more, which
-// give each of its threads a vector, and for fewer rows than this; otherwise a
-// wave per row.  A wave per row leaves two waves per SIMD at 2048 rows, too few
-// to cover the load latency.  rmsnorm_quant, wave -> block per row, us (graph
-// replay, one MI355X): 4096 wide, 256 / 512 / 1100 / 2048 / 8192 rows 5.6 / 5.9 /
-// 7.8 / 10.0 / 22.3 -> 4.1 / 4.6 / 6.4 / 9.4 / 22.2; 8192 wide 8.4 / 8.9 / 14.2 /
-// 17.0 / 46.6 -> 5.0 / 6.0 / 10.2 / 13.8 / 34.3.  srq_rmsnorm and
-// srq_rmsnorm_quant choose by the same rule, so the fused and the unfused
-// normalization round alike.
+// Rows below which a block shares each row (rmsnorm_row_kernel); above it
+// one wave per row.  srq_rmsnorm and srq_rmsnorm_quant choose by the same
+// rule, so the fused and the unfused normalization round alike.
 constexpr int64_t kRmsRowSplitRows = 256;
 
 template <bool QUANT>
 static void launch_rmsnorm_vec(const void *x, int64_t rows, int64_t nvec, float eps,
                                float mean_dim, void *out, float clip, void *q, void *qs,
                                hipStream_t st) {
-    if (rows < kRmsRowSplitRows || nvec >= 256) {
+    if (rows < kRmsRowSplitRows && nvec <= 1024) {
         auto go_row = [&](auto vt) {
             constexpr int V = decltype(vt)::value;
             rmsnorm_row_kernel<V, QUANT><<<dim3((unsigned)rows), 256, 0, st>>>(
@@ -252,7 +246,9 @@ static void launch_rmsnorm_vec(const void *x, int64_t rows, int64_t nvec, float 
     };
     if (vpt <= 1) go(std::integral_constant<int, 1>{});
     else if (vpt <= 2) go(std::integral_constant<int, 2>{});
-    else go(std::integral_constant<int, 4>{});
+    else if (vpt <= 4) go(std::integral_constant<int, 4>{});
+    else if (vpt <= 8) go(std::integral_constant<int, 8>{});
+    else go(std::integral_constant<int, 16>{});
 }
 
 extern "C" int srq_rmsnorm(const void *x, int64_t rows, int64_t cols, float eps, int64_t mean_dim,
