@@ -73,31 +73,19 @@ SRQ_DEV v16f mfma32(v8h a, v8h b, v16f c) {
 // buffer after them, so one barrier per tile covers both "tile t + 1 is in
 // LDS" and "every wave is done with the buffer tile t + 2 will overwrite",
 // and the load latency hides behind the compute.
-//
-// KSP = 2: the waves of a row group come in two sets that take the key tiles
-// alternately (two tiles staged per step), each with its own running max,
-// sum and O, merged through LDS at the end.  A block then has half the query
-// rows and half the steps, for launches whose heaviest causal q tile, not
-// the work per CU, sets the time.
-template <int NWV, int GH, int KSP = 1>
+template <int NWV, int GH>
 __global__ void __launch_bounds__(NWV * 64, 8 / NWV) prefill_attn_kernel(AttnArgs a) {
     constexpr int NT = NWV * 64;              // threads
-    constexpr int RG = NWV / (GH * KSP);      // 32-row groups
-    constexpr int QB = 32 * RG;               // query rows per block
-    static_assert(NWV % (GH * KSP) == 0 && (NT == 256 || NT == 512), "block shape");
-    constexpr int kKBytes = KSP * KT * KS * 2, kVBytes = KSP * KT * VR * 2;
-    __shared__ __align__(16) uint8_t kv_[2 * (kKBytes + kVBytes)];
-    __shared__ float kbias_[2][KSP * KT];
-    auto ks_of = [&](int buf) { return reinterpret_cast<f16 *>(kv_ + buf * kKBytes); };
-    auto vs_of = [&](int buf) {
-        return reinterpret_cast<f16 *>(kv_ + 2 * kKBytes + buf * kVBytes);
-    };
+    constexpr int QB = 32 * NWV / GH;         // query rows per block
+    static_assert(NWV % GH == 0 && (NT == 256 || NT == 512), "block shape");
+    __shared__ __align__(16) f16 Ks_[2][KT * KS];
+    __shared__ __align__(16) f16 Vs_[2][KT * VR];
+    __shared__ float kbias_[2][KT];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 5, ln = lane & 31;
-    const int rgrp = wave / GH % RG;          // this wave's 32-row group
-    const int kset = wave / (GH * RG);        // its set of key tiles
+    const int rgrp = wave / GH;               // this wave's 32-row group
     // dispatch order: the linear block id runs over the head groups fastest,
     // so under a causal mask the heaviest q tiles of every head group go
     // first and the light ones fill in behind them (with the q tile fastest,
@@ -138,20 +126,18 @@ __global__ void __launch_bounds__(NWV * 64, 8 / NWV) prefill_attn_kernel(AttnArg
 
     const int kv_end = a.causal ? min(a.T, q0 + QB) : a.T;
     const int ntiles = (kv_end + KT - 1) / KT;
-    const int nsteps = (ntiles + KSP - 1) / KSP;   // KSP tiles each
 
-    // staging registers of one step, NT threads: row tid / KR of K and of V,
-    // KH halves from (tid % KR) * KH; key bias tid (< KSP KT) (raw loads; the
+    // staging registers of one tile, NT threads: row tid / KR of K and of V,
+    // KH halves from (tid % KR) * KH; key bias tid (< KT) (raw loads; the
     // masking selects run at store time, after the MFMAs, so that no use of a
     // loaded value forces its wait before them)
-    constexpr int KTS = KSP * KT;             // keys per step
-    constexpr int KR = NT / KTS, KH = HD / KR;
+    constexpr int KR = NT / KT, KH = HD / KR;
     v8h kx[KH / 8], vx[KH / 8];
     bool ok = false;
     float kbv = 0.f;
     auto load_tile = [&](int t) __attribute__((always_inline)) {
         const int r = tid / KR, d0 = (tid % KR) * KH;
-        const int key = t * KTS + r;
+        const int key = t * KT + r;
         ok = key < a.T && (!mb || mb[key] != 0);
         const int64_t off = (int64_t)(ok ? key : 0) * a.kv_tok + d0;
 #pragma unroll
@@ -159,8 +145,8 @@ __global__ void __launch_bounds__(NWV * 64, 8 / NWV) prefill_attn_kernel(AttnArg
             kx[i] = *reinterpret_cast<const v8h *>(kb + off + 8 * i);
             vx[i] = *reinterpret_cast<const v8h *>(vb + off + 8 * i);
         }
-        if (tid < KTS) {
-            const int kz = t * KTS + tid;
+        if (tid < KT) {
+            const int kz = t * KT + tid;
             const bool live = kz < a.T && (!mb || mb[kz] != 0);
             kbv = live ? 0.f : -INFINITY;
         }
@@ -169,17 +155,17 @@ __global__ void __launch_bounds__(NWV * 64, 8 / NWV) prefill_attn_kernel(AttnArg
     auto store_tile = [&](int buf, int t) __attribute__((always_inline)) {
         // a tile with every key live (no mask, inside the sequence; uniform
         // over the block) needs no selects (T = 8192: 1376 -> 1347 us)
-        if ((mb || (t + 1) * KTS > a.T) && !ok) {
+        if ((mb || (t + 1) * KT > a.T) && !ok) {
 #pragma unroll
             for (int i = 0; i < KH / 8; ++i) kx[i] = vx[i] = (v8h)(f16)0;
         }
         const int r = tid / KR, d0 = (tid % KR) * KH;
 #pragma unroll
         for (int i = 0; i < KH / 8; ++i) {
-            *reinterpret_cast<v8h *>(ks_of(buf) + r * KS + d0 + 8 * i) = kx[i];
-            *reinterpret_cast<v8h *>(vs_of(buf) + r * VR + d0 + 8 * i) = vx[i];
+            *reinterpret_cast<v8h *>(&Ks_[buf][r * KS + d0 + 8 * i]) = kx[i];
+            *reinterpret_cast<v8h *>(&Vs_[buf][r * VR + d0 + 8 * i]) = vx[i];
         }
-        if (tid < KTS) kbias_[buf][tid] = kbv;
+        if (tid < KT) kbias_[buf][tid] = kbv;
     };
 
     if (ntiles > 0) {
@@ -187,17 +173,16 @@ __global__ void __launch_bounds__(NWV * 64, 8 / NWV) prefill_attn_kernel(AttnArg
         store_tile(0, 0);
     }
     __syncthreads();
-    for (int t = 0; t < nsteps; ++t) {
-        const int k0 = (t * KSP + kset) * KT;
+    for (int t = 0; t < ntiles; ++t) {
+        const int k0 = t * KT;
         const int buf = t & 1;
-        const f16 *Ks = ks_of(buf) + kset * KT * KS;
-        const f16 *Vs = vs_of(buf) + kset * KT * VR;
-        const float *kbias = kbias_[buf] + kset * KT;
-        if (t + 1 < nsteps) load_tile(t + 1);  // in flight during this tile's MFMAs
+        const f16 *Ks = Ks_[buf];
+        const f16 *Vs = Vs_[buf];
+        const float *kbias = kbias_[buf];
+        if (t + 1 < ntiles) load_tile(t + 1);  // in flight during this tile's MFMAs
         // this tile's compute (returns early when no key is visible)
         [&]() __attribute__((always_inline)) {
-            // no key of this tile is visible (or there is no such tile)
-            if (k0 >= kv_end || (a.causal && k0 > wave_last)) return;
+            if (a.causal && k0 > wave_last) return;   // no key of this tile is visible
 
             // S^T, two 32-key blocks
             v16f s[2];
@@ -282,36 +267,8 @@ __global__ void __launch_bounds__(NWV * 64, 8 / NWV) prefill_attn_kernel(AttnArg
                     o[db] = mfma32(av, pb[st], o[db]);
                 }
         }();
-        if (t + 1 < nsteps) store_tile(buf ^ 1, t + 1);
+        if (t + 1 < ntiles) store_tile(buf ^ 1, t + 1);
         __syncthreads();
-    }
-
-    if constexpr (KSP == 2) {
-        // the second set's states through the K/V buffers (all reads of them
-        // are done): m, l and the 64 values of O per lane, lane-major
-        constexpr int kRec = 2 + HD / 2;
-        static_assert(NWV / 2 * 64 * kRec * 4 <= 2 * (kKBytes + kVBytes), "merge area");
-        float *rec = reinterpret_cast<float *>(kv_) + (wave % (GH * RG)) * 64 * kRec + lane;
-        if (kset == 1) {
-            rec[0] = m;
-            rec[64] = l;
-#pragma unroll
-            for (int i = 0; i < HD / 32; ++i)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) rec[64 * (2 + 16 * i + v)] = o[i][v];
-        }
-        __syncthreads();
-        if (kset == 1) return;
-        const float m1 = rec[0], mm = fmaxf(m, m1);
-        // a set that saw no key has m = -inf and zeros
-        const float a0 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mm);
-        const float a1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - mm);
-        l = l * a0 + rec[64] * a1;
-#pragma unroll
-        for (int i = 0; i < HD / 32; ++i)
-#pragma unroll
-            for (int v = 0; v < 16; ++v)
-                o[i][v] = o[i][v] * a0 + rec[64 * (2 + 16 * i + v)] * a1;
     }
 
     if (qrow >= a.T) return;
@@ -384,8 +341,8 @@ extern "C" int srq_prefill_attention(const void *q, const void *k, const void *v
     // the 4-wave form: 25 against 31 us)
     hipStream_t st = (hipStream_t)stream;
     bool fits = true;
-    auto go = [&](auto kern, int nwv, int gh, int ksp = 1) {
-        const int qb = 32 * nwv / (gh * ksp);
+    auto go = [&](auto kern, int nwv, int gh) {
+        const int qb = 32 * nwv / gh;
         // the kernel's linear block id over (q tile, head group) is 32-bit
         if (srq_cdiv(seq_len, qb) * (n_q_heads / gh) >= (int64_t)1 << 31) {
             fits = false;
@@ -397,21 +354,24 @@ extern "C" int srq_prefill_attention(const void *q, const void *k, const void *v
     constexpr int64_t kCUs = 256;
     const bool gqa = (a.group == 2 || a.group == 4 || a.group == 8) &&
                      srq_cdiv(seq_len, 256 / a.group) * (n_q_heads / a.group) * batch >= kCUs;
-    // Short causal prompts with groups of 4 or 8, whose heaviest q tile sets the
-    // time: blocks of 32 rows of 4 heads, n of them.  Up to 256 tokens (or 400
-    // where two rounds of larger blocks would start) 4-wave blocks, two per
-    // CU; longer ones with the key tiles shared by two sets of waves, while n
-    // blocks run in one round (or the heaviest tile outlasts two).  us, the
-    // form below -> these (one MI355X, B x T, 32 / 64 query heads over 8):
-    //   32: 1 x 200 11.9 -> 10.9, 1 x 512 18.5 -> 17.3, 1 x 1100 34 -> 28, 1 x 1500
-    //   45 -> 36, 1 x 2048 67 -> 57, 2 x 800 36.5 -> 29; 64: 1 x 512 19.9 -> 18.1,
-    //   2 x 350 21.3 -> 18.6.  Past that more, smaller blocks lose: 32: 2 x 1100
-    //   44 against 48, 64: 2 x 512 26.4 against 28.6, 1 x 2048 92 against 108.
+    // Causal prompts without padding whose heaviest q tile sets the time (n
+    // blocks of 32 rows of 4 heads fit the CUs at once: one per CU, or two of
+    // one prompt, where a heavy block's neighbour is a light one): 4-wave
+    // blocks of 32 rows that share the staged K/V among 4 heads.  An odd number
+    // of 64-key tiles leaves half of the 128-row form's last, heaviest block
+    // empty, and that form is as fast or faster, as it is for one tile.  A
+    // row's key tiles come in the same order in every form: same bits.  us, the
+    // form below -> this (one MI355X, B x T, 32 / 64 query heads over 8):
+    //   32: 1 x 65 8.6 -> 7.6, 1 x 128 9.5 -> 8.8, 1 x 512 17.9 -> 17.2, 1 x 1100
+    //   33.3 -> 32.1, 1 x 2048 65 -> 58; 64: 1 x 512 18.9 -> 17.9, 1 x 1024 38.4 ->
+    //   34.1.  Outside the rule: one tile, 1 x 33 6.1 against 7.5; odd, 1 x 300
+    //   12.4 against 12.9; n = 496, 2 x 961 37.4 against 39.6; n = 1024, 1 x 2048 of
+    //   64 heads 85.7 against 94.1; padded, 1 x 100 9.8 against 10.1.
     const int64_t n = srq_cdiv(seq_len, 32) * (n_q_heads / 4) * batch;
-    const bool small = a.causal && a.group % 4 == 0 && n <= 2 * kCUs;
-    if (small && seq_len > 256 && (n <= kCUs || seq_len >= 700)) {
-        go(prefill_attn_kernel<8, 4, 2>, 8, 4, 2);
-    } else if (small && seq_len <= 400) {
+    const bool small = a.causal && !a.mask && a.group % 4 == 0 && seq_len > KT &&
+                       srq_cdiv(seq_len, KT) % 2 == 0 &&
+                       n <= (batch == 1 ? 2 * kCUs : kCUs);
+    if (small) {
         go(prefill_attn_kernel<4, 4>, 4, 4);
     } else switch (gqa ? a.group : 1) {
     case 2: go(prefill_attn_kernel<8, 2>, 8, 2); break;

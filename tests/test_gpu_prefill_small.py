@@ -1,7 +1,7 @@
-"""Prefill attention of short causal prompts (32-row blocks of 4 heads, and the
-form whose wave sets share the key tiles) against float32 attention: lengths
-at the edges of tiles, steps and of the rule that picks the form, groups of 4
-and 8, left padding down to one live token, strided inputs."""
+"""Prefill attention of short causal prompts (32-row blocks of 4 heads) against
+float32 attention: lengths at the edges of tiles and of the rule that picks the
+form, groups of 4 and 8, left padding down to one live token, strided inputs;
+and the same bits whatever form a prompt's batch takes."""
 import pytest
 import torch
 
@@ -49,3 +49,21 @@ def test_short_prompts(Hq, Hkv, B, T, padded):
     assert torch.allclose(out, want, rtol=4e-3, atol=4e-3)
     if mask is not None:
         assert torch.all(out[mask == 0] == 0)
+
+
+# one prompt on its own, and among others that take it out of the rule for 32-row blocks
+@pytest.mark.parametrize("Hq,Hkv", [(8, 2), (32, 8), (64, 8)])
+@pytest.mark.parametrize("T", [1, 65, 128, 257, 300, 512, 700, 1024, 2048])
+def test_same_bits_in_any_batch(Hq, Hkv, T):
+    from signrot_amd import _CUDA as C
+    gen = torch.Generator("cuda").manual_seed(T + Hq)
+    B = 1 + 512 // (-(-T // 32) * (Hq // 4)) + 1
+    q, k, v = (torch.randn(B, T, h, D, device="cuda", generator=gen).half()
+               for h in (Hq, Hkv, Hkv))
+    want = C.prefill_attention(q, k, v, None)
+    for b in {0, B - 1}:
+        got = C.prefill_attention(*(t[b:b + 1].contiguous() for t in (q, k, v)), None)
+        assert torch.equal(got[0], want[b])
+    # and with a mask that hides nothing
+    ones = torch.ones(1, T, dtype=torch.int32, device="cuda")
+    assert torch.equal(C.prefill_attention(q[:1], k[:1], v[:1], ones)[0], want[0])
