@@ -138,15 +138,19 @@ class W4A4LlamaDecodeLayer(torch.nn.Module):
             out = _CUDA.w4a4_linear_residual(qd, sd.view(-1), self.w_down, self.s_down, x2,
                                              out=x2)
             return out.view(B, 1, self.hidden)
-        gu = _CUDA.w4a4_linear(q2, s2.view(-1), self.w_gu, self.s_gu)
-        if _CUDA.swiglu_had_fusable(self.ffn, self.down_k):
-            qd, sd = _CUDA.swiglu_had_sign_quant(gu, self.down_hadk, self.down_k,
-                                                 self.down_sign)
-        else:  # no fused SwiGLU form of this rotation size
-            a = kernel.swiglu(gu[:, : self.ffn], gu[:, self.ffn:])
-            qd, sd = _CUDA.had_sign_quant(a, self.down_hadk, self.down_k, self.down_sign)
+        qd, sd = self._swiglu_rotate_quant(
+            _CUDA.w4a4_linear(q2, s2.view(-1), self.w_gu, self.s_gu))
         out = _CUDA.w4a4_linear_residual(qd, sd.view(-1), self.w_down, self.s_down, x2, out=x2)
         return out.view(B, 1, self.hidden)
+
+    def _swiglu_rotate_quant(self, gu):
+        """down_proj's codes and scales from the gate/up projection output gu
+        [R, 2 ffn], in one launch where the rotation has a SwiGLU form (which
+        addresses gu by 32-bit byte offsets)."""
+        if _CUDA.swiglu_had_fusable(self.ffn, self.down_k) and 2 * gu.numel() < 0xFFFFFFF0:
+            return _CUDA.swiglu_had_sign_quant(gu, self.down_hadk, self.down_k, self.down_sign)
+        a = kernel.swiglu(gu[:, : self.ffn], gu[:, self.ffn:])
+        return _CUDA.had_sign_quant(a, self.down_hadk, self.down_k, self.down_sign)
 
     def _forward_ops(self, hidden_states, cache, cos, sin, trace=None, attention_mask=None):
         """Op-by-op decode step (the reference's sequence of ops)."""
@@ -212,9 +216,9 @@ class W4A4LlamaDecodeLayer(torch.nn.Module):
         return self._mlp(x2, keep).view(B, T, self.hidden)
 
     def _prefill_fusable(self, h):
-        """Sizes and alignment that rmsnorm_quant, head_had_quant and the
-        SwiGLU epilogue all take (head counts below 8 have no op-by-op
-        rotation either: hadamard_transform starts at 8)."""
+        """Sizes and alignment that rmsnorm_quant, head_had_quant and the MLP's
+        kernels all take (head counts below 8 have no op-by-op rotation
+        either: hadamard_transform starts at 8)."""
         return (h.dtype == torch.float16 and h.is_cuda and h.numel() > 0
                 and h.data_ptr() % 16 == 0 and self.hidden % 8 == 0 and self.hidden <= 8192
                 and self.ffn % 8 == 0 and 8 <= self.n_heads <= 64
@@ -226,8 +230,7 @@ class W4A4LlamaDecodeLayer(torch.nn.Module):
         has to be left out of the cache, or the cache is an adapter that has
         only update()) -> prefill attention over the strided
         views -> head_had_quant -> o_proj GEMM + residual -> rmsnorm_quant ->
-        gate/up GEMM with the SwiGLU in its epilogue -> had_sign_quant -> down
-        GEMM + residual."""
+        gate/up GEMM -> swiglu_had_sign_quant -> down GEMM + residual."""
         B, T, _ = hidden_states.shape
         D, Hq, Hk = self.head_dim, self.n_heads, self.n_kv
         x2 = hidden_states.reshape(B * T, self.hidden).contiguous()
@@ -249,9 +252,14 @@ class W4A4LlamaDecodeLayer(torch.nn.Module):
         qa, sa = _CUDA.head_had_quant(attn.view(B * T, Hq, D), _inv_sqrt_f32(Hq))
         x2 = _CUDA.w4a4_linear_residual(qa, sa.view(-1), self.w_o, self.s_o, x2)
         q2, s2 = _CUDA.rmsnorm_quant(x2, n2.eps, n2.mean_dim)
-        w_il, s_il = self._gate_up_interleaved()
-        a = _CUDA.w4a4_linear_swiglu(q2, s2.view(-1), w_il, s_il)
-        qd, sd = _CUDA.had_sign_quant(a, self.down_hadk, self.down_k, self.down_sign)
+        # The weights themselves and not decode's derived copy: a prefill may be
+        # the layer's first call, on any stream or inside a graph capture, after
+        # any change of the weights, and a program that only prefills holds them
+        # once.  GEMM and swiglu_had_sign_quant at 101 / 512 / 2048 rows of 8B
+        # widths: 34 / 100 / 287 us (from the copy 29 / 85 / 252, with the copy
+        # made each time 106 / 162 / 327).
+        qd, sd = self._swiglu_rotate_quant(
+            _CUDA.w4a4_linear(q2, s2.view(-1), self.w_gu, self.s_gu))
         out = _CUDA.w4a4_linear_residual(qd, sd.view(-1), self.w_down, self.s_down, x2, out=x2)
         return out.view(B, T, self.hidden)
 

@@ -92,3 +92,54 @@ def test_prefill_through_cache_adapter():
         outs.append((layer.prefill(h, wrap(cache), cos, sin), cache.pages, cache.scales))
     for a, b in zip(*outs):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+def _prefill(layer, h, cos, sin, **cache_kw):
+    from signrot_amd.transformers import MultiLayerPagedKVCache4Bit
+    B, T, _ = h.shape
+    cache = MultiLayerPagedKVCache4Bit(B, 16, T, "cuda", 1, layer.n_kv, D,
+                                       group_size=layer.n_heads // layer.n_kv, **cache_kw)
+    return layer.prefill(h, cache, cos, sin)
+
+
+def test_prefill_reads_the_weights_themselves():
+    """A prefill keeps nothing of the weights: it follows a change that leaves
+    the tensors' version counters alone, takes buffers that have none, and
+    leaves no derived copy on the layer."""
+    layer, T = _layer(1024, 8, 2, 896), 33
+    h = torch.randn(1, T, 1024, device="cuda").half()
+    cos, sin = _cos_sin(1, T, False)
+    before = set(vars(layer))
+    _prefill(layer, h, cos, sin)
+    assert set(vars(layer)) == before
+    layer.w_gu.data.copy_(layer.w_gu.flip(0))
+    layer.s_gu.data.copy_(layer.s_gu.flip(0) * 2)
+    got = _prefill(layer, h, cos, sin)
+    fresh = _layer(1024, 8, 2, 896)
+    fresh.load_state_dict(layer.state_dict())
+    assert torch.equal(got, _prefill(fresh, h, cos, sin))
+    with torch.inference_mode():
+        inf = _layer(1024, 8, 2, 896)
+        inf.load_state_dict(layer.state_dict())
+    assert torch.equal(got, _prefill(inf, h, cos, sin))
+
+
+def test_prefill_first_in_capture_then_eager():
+    """The layer's first prefill recorded into a graph, an eager one before
+    the first replay: each computes its own."""
+    from signrot_amd.transformers import MultiLayerPagedKVCache4Bit
+    layer, T = _layer(1024, 8, 2, 896), 64
+    h = torch.randn(1, T, 1024, device="cuda").half()
+    cos, sin = _cos_sin(1, T, False)
+    want = _prefill(layer, h, cos, sin)
+    new = _layer(1024, 8, 2, 896)
+    cache = MultiLayerPagedKVCache4Bit(1, 16, T, "cuda", 1, 2, D, group_size=4)
+    cache.refresh_specs(T)
+    cache.freeze_specs(True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = new.prefill(h, cache, cos, sin)
+    assert torch.equal(_prefill(new, h, cos, sin), want)
+    for _ in range(3):
+        graph.replay()
+        assert torch.equal(out, want)
