@@ -435,14 +435,19 @@ class MultiLayerPagedKVCache4Bit(Cache):
             if T != 1:
                 raise ValueError("after the prefill, update() appends one token per request")
             raise RuntimeError("prefill: the cache already holds this layer's context")
+        length = self.length
         if layer_idx == 0:
-            self._reserve(self.length + T)
-            self.length += T
-        spec = self.get_cache_specs_for_flash_infer(None)
+            self._reserve(length + T)
+            self.length = length + T
+        try:
+            spec = self.get_cache_specs_for_flash_infer(None)
+            _CUDA.prefill_qkv_cache(qkv, cos.contiguous(), sin.contiguous(), num_q_heads, **spec,
+                                    layer_idx=layer_idx, had_scale=1 / math.sqrt(self.head_dim),
+                                    rotate=self.hadamard_dtype is not None)
+        except BaseException:   # refused (cos / sin of another shape or type): no tokens came in
+            self.length = length
+            raise
         self._filled[layer_idx] = True
-        _CUDA.prefill_qkv_cache(qkv, cos.contiguous(), sin.contiguous(), num_q_heads, **spec,
-                                layer_idx=layer_idx, had_scale=1 / math.sqrt(self.head_dim),
-                                rotate=self.hadamard_dtype is not None)
         heads = qkv.view(B, T, num_q_heads + 2 * self.num_heads, self.head_dim)
         return heads.split((num_q_heads, self.num_heads, self.num_heads), dim=2)
 

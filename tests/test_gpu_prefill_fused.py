@@ -143,3 +143,25 @@ def test_prefill_first_in_capture_then_eager():
     for _ in range(3):
         graph.replay()
         assert torch.equal(out, want)
+
+
+def test_refused_prefill_leaves_the_cache_alone():
+    """A call that is refused for its cos / sin leaves the cache as it was: the
+    corrected one then gives what a first call gives."""
+    from signrot_amd.transformers import MultiLayerPagedKVCache4Bit
+    layer, B, T = _layer(1024, 8, 2, 896), 2, 33
+    h = torch.randn(B, T, 1024, device="cuda").half()
+    cos, sin = _cos_sin(B, T, False)
+    want = _run(layer, h, B, T, 16, cos, sin, None, None)
+    cache = MultiLayerPagedKVCache4Bit(B, 16, T, "cuda", 1, 2, D, group_size=4)
+    cache.pages.zero_()
+    cache.scales.zero_()
+    for c, s in ((cos.float(), sin.float()), (cos[:, 1:], sin[:, 1:]), (cos, sin[:, 1:]),
+                 (cos.cpu(), sin.cpu()), (torch.cat([cos] * 3), torch.cat([sin] * 3))):
+        with pytest.raises(RuntimeError):
+            layer.prefill(h, cache, c, s)
+        assert cache.length == 0 and not any(cache._filled)
+    out = layer.prefill(h, cache, cos, sin)
+    assert cache.length == T
+    for a, b in zip((out, cache.pages, cache.scales), want):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
