@@ -23,6 +23,7 @@ from ..functional import kernel
 from ..functional.hadamard import _inv_sqrt_f32, get_hadK, matmul_hadU_cuda
 from ..functional.quantization import rtn_weight_pack
 from ..nn.normalization import RMSNorm
+from .kv_cache import qkv_prefill_of
 
 
 def rope_cos_sin(positions, head_dim, theta, device):
@@ -218,8 +219,16 @@ class W4A4LlamaDecodeLayer(torch.nn.Module):
     def _prefill_fusable(self, h):
         """Sizes and alignment that rmsnorm_quant, head_had_quant and the MLP's
         kernels all take (head counts below 8 have no op-by-op rotation
-        either: hadamard_transform starts at 8)."""
-        return (h.dtype == torch.float16 and h.is_cuda and h.numel() > 0
+        either: hadamard_transform starts at 8), and nothing that only calls
+        of the modules and torch's own adds would see: hooks on the norms or
+        another norm in their place, gradients of the residual stream."""
+        plain = all(type(n) is RMSNorm and "forward" not in vars(n)
+                    and not n._forward_pre_hooks and not n._forward_hooks
+                    for n in (self.input_layernorm, self.post_attention_layernorm))
+        hooked = torch.nn.modules.module._global_forward_pre_hooks or \
+            torch.nn.modules.module._global_forward_hooks
+        return (plain and not hooked and not (h.requires_grad and torch.is_grad_enabled())
+                and h.dtype == torch.float16 and h.is_cuda and h.numel() > 0
                 and h.data_ptr() % 16 == 0 and self.hidden % 8 == 0 and self.hidden <= 8192
                 and self.ffn % 8 == 0 and 8 <= self.n_heads <= 64
                 and self.n_heads & (self.n_heads - 1) == 0)
@@ -227,8 +236,8 @@ class W4A4LlamaDecodeLayer(torch.nn.Module):
     def _prefill_fused(self, hidden_states, cache, cos, sin, attention_mask):
         """rmsnorm_quant -> q/k/v GEMM -> prefill_qkv_cache (RoPE in place, K
         Hadamard, KV quantize + cache fill; the op-by-op update when padding
-        has to be left out of the cache, or the cache is an adapter that has
-        only update()) -> prefill attention over the strided
+        has to be left out of the cache, or the cache has only an update(), or
+        one of its own) -> prefill attention over the strided
         views -> head_had_quant -> o_proj GEMM + residual -> rmsnorm_quant ->
         gate/up GEMM -> swiglu_had_sign_quant -> down GEMM + residual."""
         B, T, _ = hidden_states.shape
@@ -237,7 +246,7 @@ class W4A4LlamaDecodeLayer(torch.nn.Module):
         n1, n2 = self.input_layernorm, self.post_attention_layernorm
         q1, s1 = _CUDA.rmsnorm_quant(x2, n1.eps, n1.mean_dim)
         qkv = _CUDA.w4a4_linear(q1, s1.view(-1), self.w_qkv, self.s_qkv)
-        fill = None if attention_mask is not None else getattr(cache, "update_qkv_prefill", None)
+        fill = None if attention_mask is not None else qkv_prefill_of(cache)
         if fill is not None:
             q, k, v = fill(qkv.view(B, T, -1), cos, sin, self.layer_idx, Hq)
         else:

@@ -568,6 +568,19 @@ class MultiLayerPagedKVCache4Bit(Cache):
         return self
 
 
+def qkv_prefill_of(cache):
+    """cache.update_qkv_prefill if it stands for cache.update(), else None: a
+    cache without it, or a subclass or an object that has put an update() or
+    a quantizer of its own in place of those that it stands for."""
+    fill = getattr(cache, "update_qkv_prefill", None)
+    base = MultiLayerPagedKVCache4Bit
+    if getattr(fill, "__func__", None) is base.update_qkv_prefill:
+        for name in ("update", "_quantize"):
+            if getattr(getattr(cache, name), "__func__", None) is not getattr(base, name):
+                return None
+    return fill
+
+
 class HFCacheAdapter(Cache):
     """An HF Cache that forwards to an inner cache object (kv_cache.py:
     501-520): lets a MultiLayerPagedKVCache4Bit, or any object with the same

@@ -165,3 +165,54 @@ def test_refused_prefill_leaves_the_cache_alone():
     assert cache.length == T
     for a, b in zip((out, cache.pages, cache.scales), want):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+def test_prefill_calls_what_is_put_in_place():
+    """Hooks on a norm, another norm, a cache's own update() and gradients of
+    the residual stream are seen by a prefill as by the op-by-op path."""
+    from signrot_amd.nn.normalization import RMSNorm
+    from signrot_amd.transformers import MultiLayerPagedKVCache4Bit
+    T = 33
+    h = torch.randn(1, T, 1024, device="cuda").half()
+    cos, sin = _cos_sin(1, T, False)
+    want = _prefill(_layer(1024, 8, 2, 896), h, cos, sin)
+
+    for norm in ("input_layernorm", "post_attention_layernorm"):
+        layer, seen = _layer(1024, 8, 2, 896), []
+        getattr(layer, norm).register_forward_hook(lambda m, a, out: seen.append(out.shape))
+        assert torch.equal(_prefill(layer, h, cos, sin), want) and len(seen) == 1
+        layer = _layer(1024, 8, 2, 896)
+        getattr(layer, norm).register_forward_pre_hook(lambda m, a: (a[0] * 0,))
+        assert not torch.equal(_prefill(layer, h, cos, sin), want)
+        layer = _layer(1024, 8, 2, 896)
+
+        class Double(RMSNorm):
+            def forward(self, x):
+                return super().forward(x * 2) * 0 + super().forward(x)
+        setattr(layer, norm, Double(1024))
+        assert torch.equal(_prefill(layer, h, cos, sin), want)
+        setattr(layer, norm, torch.nn.Identity())
+        assert not torch.equal(_prefill(layer, h, cos, sin), want)
+    layer, seen = _layer(1024, 8, 2, 896), []
+    handle = torch.nn.modules.module.register_module_forward_hook(
+        lambda m, a, out: seen.append(type(m)))
+    try:
+        assert torch.equal(_prefill(layer, h, cos, sin), want)
+    finally:
+        handle.remove()
+    assert seen.count(RMSNorm) == 2
+
+    calls = []
+
+    class Own(MultiLayerPagedKVCache4Bit):
+        def update(self, k, v, *a, **kw):
+            calls.append(k.shape)
+            return super().update(k, v, *a, **kw)
+    cache = Own(1, 16, T, "cuda", 1, 2, D, group_size=4)
+    assert torch.equal(layer.prefill(h, cache, cos, sin), want) and len(calls) == 1
+
+    hg = h.clone().requires_grad_()
+    out = _prefill(layer, hg, cos, sin)
+    assert torch.equal(out, want) and out.requires_grad
+    out.float().sum().backward()
+    assert torch.equal(hg.grad, torch.ones_like(hg))   # through the residual adds
