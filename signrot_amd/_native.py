@@ -135,6 +135,8 @@ class _HostOps:
     any other, which the Python op then handles."""
 
     def __getattr__(self, name):
+        if name.startswith("_"):
+            raise AttributeError(name)
         lib()
         if not HOST_PATH.exists():
             raise RuntimeError(
@@ -145,6 +147,8 @@ class _HostOps:
         mod = importlib.util.module_from_spec(spec)
         loader.exec_module(mod)
         self.__dict__.update({k: f for k, f in vars(mod).items() if not k.startswith("_")})
+        if name not in self.__dict__:
+            raise AttributeError(f"srq_host has no op {name!r}")
         return self.__dict__[name]
 
 

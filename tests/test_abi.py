@@ -117,3 +117,14 @@ def test_asym_argument_errors(lib):
     assert lib.srq_sum_i4(None, 0, 16, 1, None, None) == 0
     assert lib.srq_matmul_colrow_i8_i32(None, None, 0, 8, None, None) == 0
     assert lib.srq_asym_quant(None, None, None, 0, 8, 0, None, None) == 0
+
+
+def test_host_ops_unknown_name():
+    """A name that the host extension does not have is an AttributeError."""
+    import torch  # noqa: F401  (the extension links against it)
+    from signrot_amd import _native
+    for ops in (_native.host, type(_native.host)()):
+        assert not hasattr(ops, "no_such_op") and not hasattr(ops, "__wrapped__")
+        with pytest.raises(AttributeError, match="no_such_op"):
+            ops.no_such_op
+        assert callable(ops.w4a4_linear) and ops.w4a4_linear() is None
