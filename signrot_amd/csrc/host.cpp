@@ -7,11 +7,14 @@
 //
 // Every function returns the op's outputs, or None for any argument that it
 // does not take as it stands (another dtype, device or shape, a view that is
-// not contiguous, a tensor subclass with its own dispatch, an error code of
-// the library): the Python op then goes through its own checks, which name
-// what is wrong, so the set of accepted calls and the errors are the Python
-// ops' own.  Outputs come from torch's caching allocator, launches go to the
-// current stream of the tensors' device, nothing synchronises.
+// not contiguous, a tensor subclass with its own dispatch, an argument that
+// the library refuses): the Python op then goes through its own checks, which
+// name what is wrong, so the set of accepted calls and the errors are the
+// Python ops' own.  None means that nothing was launched: a failed launch is
+// raised here, as the Python op raises it (the kernel may have run, and an
+// in-place residual must not be added twice).  Outputs come from torch's
+// caching allocator, launches go to the current stream of the tensors' device,
+// nothing synchronises.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -24,7 +27,8 @@
 
 namespace {
 
-struct Bad {};  // an argument this file does not take
+struct Bad {};     // an argument this file does not take
+struct Raised {};  // a Python exception is set
 
 // the interpreter lock is not held while allocating and launching
 struct NoGil {
@@ -92,13 +96,39 @@ c10::SmallVector<int64_t, 6> with_last(const at::Tensor &x, int64_t last) {
     return s;
 }
 
+// The library's answer: nothing for success, Bad for arguments that it refuses
+// (its entry points check them before any launch), else the exception that
+// _native.call raises.
+void check(int rc, const char *entry) {
+    if (rc == SRQ_OK) return;
+    if (rc == SRQ_EINVAL || rc == SRQ_EUNSUPPORTED) throw Bad();
+    PyObject *mod = PyImport_ImportModule("signrot_amd._native");
+    PyObject *type = mod ? PyObject_GetAttrString(mod, "NativeError") : nullptr;
+    if (type) PyErr_Format(type, "%s failed (%d): %s", entry, rc, srq_last_error());
+    Py_XDECREF(type);
+    Py_XDECREF(mod);
+    throw Raised();
+}
+
+// The outputs of an op that has run: an error in here is raised.
 PyObject *wrap(std::initializer_list<at::Tensor> ts) {
-    if (ts.size() == 1) return THPVariable_Wrap(*ts.begin());
-    PyObject *r = PyTuple_New((Py_ssize_t)ts.size());
-    if (!r) return nullptr;
-    Py_ssize_t i = 0;
-    for (const at::Tensor &t : ts) PyTuple_SET_ITEM(r, i++, THPVariable_Wrap(t));
-    return r;
+    PyObject *r = nullptr;
+    try {
+        if (ts.size() == 1) return THPVariable_Wrap(*ts.begin());
+        r = PyTuple_New((Py_ssize_t)ts.size());
+        if (!r) throw Raised();
+        Py_ssize_t i = 0;
+        for (const at::Tensor &t : ts) {
+            PyObject *o = THPVariable_Wrap(t);
+            if (!o) throw Raised();
+            PyTuple_SET_ITEM(r, i++, o);
+        }
+        return r;
+    } catch (...) {
+        Py_XDECREF(r);
+        if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "srq_host: output not wrapped");
+        throw Raised();
+    }
 }
 
 // Runs one op's body; anything it does not take becomes None.
@@ -107,6 +137,8 @@ PyObject *guarded(Py_ssize_t have, Py_ssize_t want, F body) {
     try {
         if (have != want) throw Bad();
         return body();
+    } catch (const Raised &) {
+        return nullptr;
     } catch (...) {
         PyErr_Clear();
         Py_RETURN_NONE;
@@ -154,7 +186,7 @@ PyObject *had_sign_quant(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
             rc = srq_had_sign_quant(x.data_ptr(), rows, n, K, h, (const int8_t *)s, f32 ? 1 : 0,
                                     clip, q.data_ptr(), sc.data_ptr(), stream_of(dev));
         }
-        if (rc) throw Bad();
+        check(rc, "srq_had_sign_quant");
         return wrap({q, sc});
     });
 }
@@ -183,7 +215,7 @@ PyObject *had_sign_asym_quant(PyObject *, PyObject *const *a, Py_ssize_t n_args)
                                               clip, q.data_ptr(), sc.data_ptr(), z.data_ptr(),
                                               stream_of(dev));
         }
-        if (rc) throw Bad();
+        check(rc, i8 ? "srq_had_sign_asym_quant_i8" : "srq_had_sign_asym_quant");
         return wrap({q, sc, z});
     });
 }
@@ -207,7 +239,7 @@ PyObject *sym_quant_dynamic(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
             rc = srq_sym_quant_dynamic(x.data_ptr(), rows, n, clip, q.data_ptr(), sc.data_ptr(),
                                        stream_of(dev));
         }
-        if (rc) throw Bad();
+        check(rc, "srq_sym_quant_dynamic");
         return wrap({q, sc});
     });
 }
@@ -229,7 +261,7 @@ PyObject *rmsnorm_quant(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
             rc = srq_rmsnorm_quant(x.data_ptr(), rows, n, eps, mean_dim, clip, nullptr,
                                    q.data_ptr(), sc.data_ptr(), stream_of(dev));
         }
-        if (rc) throw Bad();
+        check(rc, "srq_rmsnorm_quant");
         return wrap({q, sc});
     });
 }
@@ -251,7 +283,7 @@ PyObject *head_had_quant(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
             rc = srq_head_had_quant(x.data_ptr(), B, H, D, scale, clip, q.data_ptr(),
                                     sc.data_ptr(), nullptr, stream_of(dev));
         }
-        if (rc) throw Bad();
+        check(rc, "srq_head_had_quant");
         return wrap({q, sc});
     });
 }
@@ -297,7 +329,7 @@ PyObject *w4a4_linear(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
             }
             ws.reset();
         }
-        if (rc) throw Bad();
+        check(rc, "srq_w4a4_linear");
         return wrap({out});
     });
 }
@@ -329,7 +361,7 @@ PyObject *w4a4_linear_residual(PyObject *, PyObject *const *a, Py_ssize_t n_args
             }
             ws.reset();
         }
-        if (rc) throw Bad();
+        check(rc, "srq_w4a4_linear_residual");
         if (given) {
             Py_INCREF(a[6]);
             return a[6];
@@ -360,7 +392,7 @@ PyObject *w4a4_linear_asym(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
                                          wb > 0 ? wb : 0, stream_of(o.dev));
             ws.reset();
         }
-        if (rc) throw Bad();
+        check(rc, "srq_w4a4_linear_asym");
         return wrap({out});
     });
 }
@@ -379,7 +411,7 @@ PyObject *w4a4_linear_swiglu(PyObject *, PyObject *const *a, Py_ssize_t n_args) 
             rc = srq_w4a4_linear_swiglu(o.A.data_ptr(), sa, o.B.data_ptr(), sb, o.M, o.N, o.K,
                                         out.data_ptr(), stream_of(o.dev));
         }
-        if (rc) throw Bad();
+        check(rc, "srq_w4a4_linear_swiglu");
         return wrap({out});
     });
 }

@@ -158,3 +158,78 @@ def test_current_stream():
         done.record(side)
     done.synchronize()
     assert torch.equal(q, want)
+
+
+_STUB = """
+int stub_rc = 0, stub_calls = 0;
+%s
+long long srq_w4a4_linear_ws_bytes() { return 0; }
+const char *srq_last_error() { return "stub"; }
+"""
+
+_CHILD = """
+import ctypes, importlib.machinery, importlib.util, pathlib, sys
+import torch
+from signrot_amd import _native
+from signrot_amd._native import NativeError
+here = pathlib.Path(sys.argv[1])
+stub = ctypes.CDLL(str(here / "libsignrot_hip.so"), mode=ctypes.RTLD_GLOBAL)
+rc, calls = (ctypes.c_int.in_dll(stub, n) for n in ("stub_rc", "stub_calls"))
+loader = importlib.machinery.ExtensionFileLoader("srq_host", str(here / "srq_host.so"))
+host = importlib.util.module_from_spec(importlib.util.spec_from_loader("srq_host", loader))
+loader.exec_module(host)
+u8 = lambda *s: torch.zeros(s, dtype=torch.uint8, device="cuda")
+f16 = lambda *s: torch.zeros(s, dtype=torch.float16, device="cuda")
+i8 = torch.zeros(2, dtype=torch.int8, device="cuda")
+i32 = torch.zeros(32, dtype=torch.int32, device="cuda")
+res = f16(2, 32)
+ops = [(host.had_sign_quant, (f16(2, 64), None, 1, None, 1.0, False)),
+       (host.had_sign_asym_quant, (f16(2, 64), None, 1, None, 1.0, True)),
+       (host.had_sign_asym_quant, (f16(2, 64), None, 1, None, 1.0, False)),
+       (host.sym_quant_dynamic, (f16(2, 64), 1.0, 2)),
+       (host.rmsnorm_quant, (f16(2, 64), 1e-5, 64, 1.0)),
+       (host.head_had_quant, (f16(2, 8, 16), 1.0, 1.0)),
+       (host.w4a4_linear, (u8(2, 32), f16(2), u8(32, 32), f16(32), None, 2)),
+       (host.w4a4_linear_residual, (u8(2, 32), f16(2), u8(32, 32), f16(32), res, None, res)),
+       (host.w4a4_linear_asym, (u8(2, 32), f16(2), i8, u8(32, 32), f16(32), i32, None, 2)),
+       (host.w4a4_linear_swiglu, (u8(2, 32), f16(2), u8(32, 32), f16(32)))]
+for op, args in ops:
+    name = op.__name__
+    for code, outcome in ((0, "result"), (-1, None), (-2, None), (-3, "raises"), (-9, "raises")):
+        rc.value, before = code, calls.value
+        try:
+            got = op(*args)
+            got = None if got is None else "result"
+        except NativeError as e:
+            got = "raises"
+            assert f"({code}): stub" in str(e) and name in str(e), (name, str(e))
+        assert got == outcome, (name, code, got)
+        assert calls.value == before + 1, (name, code)
+print("ok", flush=True)
+"""
+
+
+def test_failed_launch_is_raised_once(tmp_path):
+    """A launch error of the library is raised and the call not repeated by
+    the Python op (an in-place residual would be added twice); an argument
+    that the library refuses goes to the Python op.  The real extension over a
+    stub of the library that only counts calls: nothing runs on the GPU."""
+    import pathlib
+    import shutil
+    import subprocess
+    import sys
+
+    import signrot_amd
+    from signrot_amd import _native
+    root = pathlib.Path(signrot_amd.__file__).resolve().parents[1]
+    entries = sorted(set(_native.SIGNATURES))
+    (tmp_path / "stub.c").write_text(_STUB % "\n".join(
+        f"int {n}() {{ ++stub_calls; return stub_rc; }}" for n in entries))
+    subprocess.run(["gcc", "-shared", "-fPIC", "-w", "-o", str(tmp_path / "libsignrot_hip.so"),
+                    str(tmp_path / "stub.c")], check=True)
+    shutil.copy(_native.HOST_PATH, tmp_path / "srq_host.so")
+    (tmp_path / "child.py").write_text(_CHILD)
+    run = subprocess.run([sys.executable, str(tmp_path / "child.py"), str(tmp_path)], cwd=root,
+                         env={**__import__("os").environ, "PYTHONPATH": str(root)},
+                         capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0 and run.stdout.strip().endswith("ok"), run.stderr[-2000:]
