@@ -37,8 +37,10 @@ struct NoGil {
     ~NoGil() { PyEval_RestoreThread(s); }
 };
 
+// a torch.Tensor or Parameter itself: a subclass may see every attribute and
+// call that the Python op makes of it
 const at::Tensor &plain(PyObject *o, at::ScalarType dt) {
-    if (!THPVariable_Check(o)) throw Bad();
+    if (!THPVariable_CheckExact(o)) throw Bad();
     const at::Tensor &t = THPVariable_Unpack(o);
     if (!t.defined() || !t.is_cuda() || t.layout() != at::kStrided || t.scalar_type() != dt ||
         !t.has_storage() || !t.is_contiguous() || t.is_neg() || t.is_conj() ||

@@ -160,6 +160,88 @@ def test_current_stream():
     assert torch.equal(q, want)
 
 
+class _Recorder:
+    """The real host ops, each call and whether it was taken noted."""
+
+    def __init__(self, ops):
+        self.ops, self.taken = ops, []
+
+    def __getattr__(self, name):
+        op = getattr(self.ops, name)
+
+        def call(*a):
+            out = op(*a)
+            if name != "stream":
+                self.taken.append(out is not None)
+            return out
+        return call
+
+
+def test_taken_and_handed_back(monkeypatch):
+    """The C++ op takes each call of _calls() at once, and none of those that
+    need a second look: subclasses, functorch wrappers, fake tensors, views
+    that are not contiguous, other scalars."""
+    import numpy as np
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from signrot_amd import _CUDA as C
+    from signrot_amd.functional import kernel
+    rec = _Recorder(C._host)
+    monkeypatch.setattr(C, "_host", rec)
+    n = 0
+    for name, call in _calls():
+        rec.taken.clear()
+        call()
+        assert rec.taken == [True], name
+        n += 1
+    assert n == 54
+
+    seen = []
+
+    class Sub(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            seen.append(func)
+            return super().__torch_function__(func, types, args, kwargs or {})
+    x = _x(4, 512)
+    a, sa, w, ws = _codes(4, 256), _scale(4), _codes(32, 256), _scale(32)
+    host = rec.ops
+    assert host.sym_quant_dynamic(torch.nn.Parameter(x), 1.0, 2) is not None
+    handed = [lambda: host.sym_quant_dynamic(x.as_subclass(Sub), 1.0, 2),
+              lambda: host.w4a4_linear(a, sa, w.as_subclass(Sub), ws, None, 2),
+              lambda: host.w4a4_linear(a, sa, w, ws, _x(32).as_subclass(Sub), 2),
+              lambda: host.sym_quant_dynamic(x.t(), 1.0, 2),
+              lambda: host.sym_quant_dynamic(x[:, ::2], 1.0, 2),
+              lambda: host.sym_quant_dynamic(x.cpu(), 1.0, 2),
+              lambda: host.sym_quant_dynamic(x.float(), 1.0, 2),
+              lambda: host.sym_quant_dynamic(x, np.float32(1.0), 2),
+              lambda: host.sym_quant_dynamic(x, torch.ones(()), 2),
+              lambda: host.sym_quant_dynamic(x, 1.0, 3),
+              lambda: host.sym_quant_dynamic(x, 1.0),
+              lambda: host.sym_quant_dynamic(None, 1.0, 2),
+              lambda: host.sym_quant_dynamic(x[:0], 1.0, 2),
+              lambda: host.sym_quant_dynamic(x.to_sparse(), 1.0, 2),
+              lambda: host.had_sign_quant(x, None, 12, None, 1.0, False),
+              lambda: host.had_sign_quant(x, None, 1, None, 1.0, 0),
+              lambda: host.w4a4_linear(a, sa[:3], w, ws, None, 2),
+              lambda: host.w4a4_linear(_codes(4, 8), sa, _codes(32, 8), ws, None, 2),
+              lambda: host.w4a4_linear_residual(a, sa, w, ws, _x(4, 31), None, None)]
+    for i, call in enumerate(handed):
+        assert call() is None, i
+    out = []
+    torch.func.vmap(lambda t: out.append(host.sym_quant_dynamic(t, 1.0, 2)) or t)(_x(2, 4, 512))
+    torch.func.grad(lambda t: out.append(host.sym_quant_dynamic(t, 1.0, 2)) or t.sum())(x)
+    torch.func.functionalize(
+        lambda t: out.append(host.sym_quant_dynamic(t, 1.0, 2)) or t)(x)
+    with FakeTensorMode():
+        out.append(host.sym_quant_dynamic(torch.empty(4, 512, device=DEV).half(), 1.0, 2))
+    assert out == [None] * 4
+    # the Python op then sees what it always saw
+    seen.clear()
+    q, s = kernel.sym_quant_dynamic(x.as_subclass(Sub))
+    assert seen and torch.equal(q, host.sym_quant_dynamic(x, 1.0, 2)[0])
+
+
 _STUB = """
 int stub_rc = 0, stub_calls = 0;
 %s
