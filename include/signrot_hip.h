@@ -112,10 +112,10 @@ int srq_w4a4_linear_swiglu(const void *A, const void *a_scale, const void *B,
                            void *stream);
 
 /* Workspace form of srq_w4a4_linear (and of srq_w4a4_linear_residual
- * below, with residual): bit-identical outputs.  For mid-size M (65 ..
+ * below, with residual): bit-identical outputs.  For mid-size M (33 ..
  * 1023) whose output tiles are too few to fill the GPU (under 192 of
  * 128 x 128, or 64 or 128 of 256 x 128 with K chunks of at least 4096
- * codes), the product is split over K into int32 partials in `workspace` (device
+ * codes, past M = 512 of 12288), the product is split over K into int32 partials in `workspace` (device
  * memory, srq_w4a4_linear_ws_bytes(M, N, K) bytes, 0 when the shape is not
  * split) and summed by a second pass before the epilogue; with a smaller
  * workspace the call runs as srq_w4a4_linear.  No counterpart in the
@@ -153,10 +153,12 @@ int srq_w4a4_linear_asym(const void *A, const void *a_scale, const int8_t *a_zer
                          const void *bias, int64_t M, int64_t N, int64_t K, void *out,
                          void *stream);
 
-/* srq_w4a4_linear_asym with a caller-owned workspace of
- * srq_w4a4_linear_ws_bytes(M, N, K) bytes (16-byte aligned; null or smaller:
- * the plain form): mid-size M with few output tiles is split over K into
- * int32 partials.  Bit-identical to srq_w4a4_linear_asym. */
+/* srq_w4a4_linear_asym with a caller-owned workspace of the bytes that
+ * srq_w4a4_linear_asym_ws_bytes writes to *bytes (0: not split; 16-byte
+ * aligned; null or smaller: the plain form): mid-size M with few output tiles
+ * and a long K is split over K into int32 partials.  Bit-identical to
+ * srq_w4a4_linear_asym. */
+int srq_w4a4_linear_asym_ws_bytes(int64_t M, int64_t N, int64_t K, int64_t *bytes);
 int srq_w4a4_linear_asym_ws(const void *A, const void *a_scale, const int8_t *a_zero,
                             const void *B, const void *b_scale, const int32_t *b_sum,
                             const void *bias, int64_t M, int64_t N, int64_t K, void *out,

@@ -25,6 +25,7 @@ Added ops (no reference counterpart, fused forms of reference chains):
   qkv_decode_i4         = qkv_rope_had_append + batch_decode_i4 kv_cache.py:144-170, 295-415
   prefill_qkv_cache     = rope_qk + K Hadamard + kv_quant_pack + init_kv_i4 kv_cache.py:295-395
 """
+import ctypes
 import functools
 
 import torch
@@ -117,7 +118,7 @@ def w4a4_linear_asym(A, a_scale, a_zero, B, b_scale, b_sum, bias=None):
     if bias is not None and bias.numel() != N:
         raise RuntimeError("w4a4_linear_asym: bias must have N elements")
     out = torch.empty((M, N), dtype=torch.float16, device=A.device)
-    ws = _splitk_workspace(M, N, K, A.device)
+    ws = _splitk_workspace(M, N, K, A.device, asym=True)
     if ws is None:
         _call("srq_w4a4_linear_asym", _ptr(A), _ptr(a_scale), _ptr(a_zero), _ptr(B),
               _ptr(b_scale), _ptr(b_sum), _ptr(bias), M, N, K, _ptr(out), _stream(A))
@@ -190,15 +191,19 @@ def w4a4_linear_swiglu(A, a_scale, B_il, b_scale_il):
 
 
 @functools.lru_cache(maxsize=512)
-def _splitk_bytes(M, N, K):
+def _splitk_bytes(M, N, K, asym=False):
+    if asym:
+        n = ctypes.c_int64()
+        _call("srq_w4a4_linear_asym_ws_bytes", M, N, K, ctypes.byref(n))
+        return n.value
     return int(_native.lib().srq_w4a4_linear_ws_bytes(M, N, K))
 
 
-def _splitk_workspace(M, N, K, device):
+def _splitk_workspace(M, N, K, device, asym=False):
     """The int32 split-K partials' workspace the library asks for at this
     shape (mid-size M with too few output tiles to fill the GPU), from
     torch's caching allocator (graph-capture safe), or None."""
-    n = _splitk_bytes(M, N, K)
+    n = _splitk_bytes(M, N, K, asym)
     return torch.empty(n, dtype=torch.uint8, device=device) if n else None
 
 

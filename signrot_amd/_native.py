@@ -33,6 +33,7 @@ SIGNATURES = {
                                     _p],
     "srq_matmul_u4s4": [_p, _p, _i64, _i64, _i64, _p, _p],
     "srq_w4a4_linear_asym": [_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p],
+    "srq_w4a4_linear_asym_ws_bytes": [_i64, _i64, _i64, _p],
     "srq_w4a4_linear_asym_ws": [_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _p, _p, _i64,
                                 _p],
     "srq_w4a4_linear_moe_asym": [_p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _p, _p],

@@ -2242,25 +2242,52 @@ struct SplitK {
 bool dense_rows(int64_t M, int64_t N, int64_t K, bool swiglu) {
     if (M <= 32 || M > 192 || K < 256) return false;
     const int64_t ct = srq_cdiv(N, kRowsBN);
+    // short K and a last round of the CUs that is nearly empty (SwiGLU over N =
+    // 36864, 288 tiles, K = 512: M = 129 / 161 19.8 / 21.6 against 21.9 / 23.6)
+    if (swiglu && K <= 1024 && ct > 256 && ct % 256 != 0 && ct % 256 <= 64) return false;
     if (M <= 96) return ct >= (swiglu ? 96 : 192);
     if (M <= 128) return swiglu && ct >= 96 && ct < 192;
     return ct >= (swiglu ? 160 : 192);
 }
-SplitK splitk_plan(int64_t M, int64_t N, int64_t K, bool fp16_out) {
+// Whether a linear of asymmetric activations takes the split-K plan of its
+// shape.  Its unsplit ring kernel is as fast as the symmetric one, and where
+// its tiles run in one round of the CUs the split's partials and second launch
+// only pay with a long K.  us unsplit / split: N = 4096, M = 256, K = 4096 / 8192 /
+// 10240 15.3 / 24.2 / 29 against 21.3 / 25.5 / 26; M = 128, K = 8960 / 10240 19.2 / 21
+// against 21.7 / 21; M = 512, K = 4096 / 8192 21.5 / 34 against 29 / 32; N = 5120,
+// M = 192, K = 4096 15.3 against 21.4.  In two rounds the split wins at any K:
+// N = 6144, M = 192, K = 4096 27.4 against 22.6.
+bool asym_split_pays(int64_t M, int64_t N, int64_t K) {
+    const int64_t bm = M <= 256 ? 64 : 128, bn = M <= 128 ? 32 : 64;   // its tiles
+    return srq_cdiv(M, bm) * srq_cdiv(N, bn) > 256 || K >= (M <= 256 ? 10240 : 8192);
+}
+
+// ua: asymmetric activations
+SplitK splitk_plan(int64_t M, int64_t N, int64_t K, bool fp16_out, bool ua) {
     SplitK p;
     if (!fp16_out || M <= 32 || M >= 1024 || K < 2048) return p;
+    if (ua && M > 64 && !asym_split_pays(M, N, K)) return p;
+    const int64_t ct = srq_cdiv(N, kRowsBN);
     // Few column tiles: all rows in one gemm_rows_kernel tile, K in S chunks
     // that give 160 to 256 tiles.  Up to 96 rows with chunks of at least 1280
     // codes, M = 33 / 64 / 96: N = 4096, K = 14336 22 / 24 / 20.6 -> 15.6 / 17 /
     // 19.8 us; N = 8192, K = 28672 67 / 75 / 44 -> 31 / 36 / 42 (N = 4096 or
-    // 6144 at K = 4096 lose: 8 against 12, 11.2 against 12.6).  Between 129
-    // and 192 rows only long chunks pay for the wider partials: M = 137 / 180
-    // at N = 8192, K = 28672 67 / 68 -> 55 / 58, but at N = 4096, K = 14336
-    // 24.6 / 25.6 against 24.8 / 27.3.
-    if (!dense_rows(M, N, K, false) && (M <= 96 || (M > 128 && M <= 192))) {
-        const int64_t ct = srq_cdiv(N, kRowsBN);
-        const int64_t S = std::min<int64_t>(256 / ct, K / (M <= 96 ? 1280 : 4096));
-        if (S >= 2 && ct * S >= 160) {
+    // 6144 at K = 4096 lose: 8 against 12, 11.2 against 12.6).  Up to 64 rows
+    // only where the skinny kernel (a block per 16 columns) has more than 8192
+    // codes of K per CU to go through: M = 33, N = 8192, K = 4096 and N = 4096, K =
+    // 8192 12.3 and 13.8 against 14.0 and 14.8; N = 5120, K = 5120 15.0 -> 13.4.
+    const bool few = M <= 96 && (M > 64 || srq_cdiv(srq_cdiv(N, 16), 256) * K > 8192);
+    // Between 129 and 192 rows only long chunks pay for the wider partials,
+    // M = 160 / 192: N = 8192, K = 28672 65 / 64.5 -> 53.5 / 58.5, N = 4096, K =
+    // 28672 38.6 / 39.3 -> 36.5 / 38.4; and tiles for 200 CUs where the 128-row
+    // tiles split well (N = 4096, K = 20480, 160 tiles: 31.5 / 32.1 against 33.0 /
+    // 34.2; they do not between 65 and 95 column tiles: N = 10240, K = 8192 43.8 ->
+    // 31.5), at most 160 rows where those fill the CUs unsplit (N = 14336, K =
+    // 8192: 36.8 / 37.3 against 36.8 / 40.5).
+    const bool wide = M > 128 && M <= (ct >= 96 ? 160 : 192);
+    if (!dense_rows(M, N, K, false) && (few || wide)) {
+        const int64_t S = std::min<int64_t>(256 / ct, K / (few ? 1280 : 4096));
+        if (S >= 2 && ct * S >= (wide && ct <= 64 ? 200 : 160)) {
             p.Kc = srq_cdiv(srq_cdiv(K, S), 256) * 256;
             p.S = (int)srq_cdiv(K, p.Kc);
             p.rows = true;
@@ -2270,12 +2297,15 @@ SplitK splitk_plan(int64_t M, int64_t N, int64_t K, bool fp16_out) {
     if (M <= 64) return p;
     const int64_t tiles = srq_cdiv(M, kGrpBM) * srq_cdiv(N, kGrpBN);
     const int64_t big = srq_cdiv(M, kBigBM) * srq_cdiv(N, kBigBN);
-    // Past M = 512 only with chunks of 12288 codes: M = 1000 / 800, N = 4096, K =
-    // 14336 (two chunks of 7168) 57.7 / 54.1 us unsplit on the dense grouped
-    // form against 62.9 / 59.1 split; M = 512, N = 8192, K = 28672 112 against
-    // 106.
+    // Past M = 512, and with asymmetric activations (whose unsplit form is the
+    // faster one), only with chunks of 12288 codes.  M = 800 / 1000, N = 4096,
+    // split in two -> unsplit on the dense grouped form: K = 8192 44 / 47 -> 35 /
+    // 37.5; 11008 53 / 56 -> 45 / 48; 14336 59 / 63 -> 54 / 58.  M = 512, N = 8192,
+    // K = 28672: 112 unsplit, 106 split; asymmetric, M = 384 / 512, N = 8192, K =
+    // 8192 40 / 43 against 48 / 53, K = 20480 80 / 89 against 87 / 93, K = 28672 105 /
+    // 120 against 105 / 118.
     if (tiles >= 192 && big >= 64 && big <= 128 && 256 % big == 0 &&
-        K / (256 / big) >= (M <= 512 ? 4096 : 12288)) {
+        K / (256 / big) >= (M <= 512 && !ua ? 4096 : 12288)) {
         // enough 128 x 128 tiles for the dense grouped form, but 256 / big
         // K-chunks of 256 x 128 tiles cover the CUs exactly, and the bigger
         // tile unpacks fewer nibbles per MFMA (the grouped kernel's compute
@@ -2296,8 +2326,9 @@ SplitK splitk_plan(int64_t M, int64_t N, int64_t K, bool fp16_out) {
     if (p.S < 2) p.S = 0;
     return p;
 }
-int64_t splitk_bytes(int64_t M, int64_t N, int64_t K, bool fp16_out) {
-    const SplitK p = splitk_plan(M, N, K, fp16_out);
+int64_t splitk_bytes(int64_t M, int64_t N, int64_t K, bool ua) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const SplitK p = splitk_plan(M, N, K, true, ua);
     return p.S ? (int64_t)p.S * M * N * 4 : 0;
 }
 
@@ -2357,7 +2388,7 @@ GroupedArgs dense_args(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N,
 template <bool UA>
 void launch_gemm(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64_t K,
                  const Epi &e, hipStream_t st, void *ws = nullptr, int64_t ws_bytes = 0) {
-    const SplitK sk = ws ? splitk_plan(M, N, K, !e.C) : SplitK{};
+    const SplitK sk = ws ? splitk_plan(M, N, K, !e.C, UA) : SplitK{};
     if (K == 0) {
         const int64_t blocks = std::min<int64_t>(srq_cdiv(M * N, 256), 4096);
         fill_zero_epilogue<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(M, N, e);
@@ -2577,8 +2608,13 @@ extern "C" int srq_w4a4_linear_swiglu(const void *A, const void *a_scale, const 
 }
 
 extern "C" int64_t srq_w4a4_linear_ws_bytes(int64_t M, int64_t N, int64_t K) {
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
-    return splitk_bytes(M, N, K, true);
+    return splitk_bytes(M, N, K, false);
+}
+
+extern "C" int srq_w4a4_linear_asym_ws_bytes(int64_t M, int64_t N, int64_t K, int64_t *bytes) {
+    SRQ_CHECK_ARG(bytes, "w4a4_linear_asym_ws_bytes: null pointer");
+    *bytes = splitk_bytes(M, N, K, true);
+    return SRQ_OK;
 }
 
 extern "C" int srq_w4a4_linear_ws(const void *A, const void *a_scale, const void *B,

@@ -386,7 +386,8 @@ PyObject *w4a4_linear_asym(PyObject *, PyObject *const *a, Py_ssize_t n_args) {
         {
             NoGil nogil;
             out = alloc(with_last(o.A, o.N), kF16, o.dev);
-            const int64_t wb = srq_w4a4_linear_ws_bytes(o.M, o.N, o.K);
+            int64_t wb = 0;
+            srq_w4a4_linear_asym_ws_bytes(o.M, o.N, o.K, &wb);
             if (wb > 0) ws = alloc({wb}, kU8, o.dev);
             rc = srq_w4a4_linear_asym_ws(o.A.data_ptr(), sa, (const int8_t *)za, o.B.data_ptr(),
                                          sb, (const int32_t *)wsum, bias, o.M, o.N, o.K,

@@ -128,3 +128,21 @@ def test_host_ops_unknown_name():
         with pytest.raises(AttributeError, match="no_such_op"):
             ops.no_such_op
         assert callable(ops.w4a4_linear) and ops.w4a4_linear() is None
+
+
+# K chunks that a linear is split into, symmetric and asymmetric activations (0:
+# one kernel), on both sides of each line of the rule
+@pytest.mark.parametrize("M,N,K,sym,asym", [
+    (33, 8192, 4096, 0, 0), (64, 4096, 8192, 0, 0),        # the skinny kernel's 8192 codes a CU
+    (33, 5120, 5120, 4, 4), (64, 4096, 10240, 8, 8), (65, 8192, 4096, 3, 3),
+    (160, 4096, 20480, 4, 4), (160, 4096, 28672, 7, 7),    # 129 to 192 rows
+    (160, 14336, 8192, 2, 2), (161, 14336, 8192, 0, 0), (192, 10240, 8192, 2, 2),
+    (128, 4096, 8960, 5, 0), (128, 4096, 10240, 5, 5),     # asymmetric, one round unsplit
+    (256, 4096, 8192, 4, 0), (256, 4096, 11008, 4, 4), (512, 4096, 4096, 2, 0),
+    (512, 4096, 8192, 2, 2), (192, 6144, 4096, 2, 2),      # two rounds
+    (512, 8192, 14336, 2, 0), (512, 8192, 28672, 2, 2),    # 256 x 128 tiles
+    (800, 4096, 14336, 0, 0), (800, 4096, 24576, 2, 2)])
+def test_split_plan(M, N, K, sym, asym):
+    from signrot_amd import _CUDA
+    got = tuple(_CUDA._splitk_bytes(M, N, K, a) / (4 * M * N) for a in (False, True))
+    assert got == (sym, asym)
