@@ -1500,7 +1500,9 @@ SRQ_DEV int64_t uni(int64_t v) {
                      (uint32_t)__builtin_amdgcn_readfirstlane((int)v));
 }
 
-template <int FORM>
+// REM: with skip_rem, an expert's leftover rows apart (xrows); without, all of
+// its rows are tiled
+template <int FORM, bool REM = true>
 SRQ_DEV GroupedProb grouped_prob(const GroupedArgs &g, int p) {
     GroupedProb r;
     r.xrows = 0;
@@ -1544,7 +1546,7 @@ SRQ_DEV GroupedProb grouped_prob(const GroupedArgs &g, int p) {
         const int e = g.pair ? p >> 1 : p;
         r.row0 = uni(g.offsets[e]);
         r.m = uni(g.offsets[e + 1]) - r.row0;
-        if (g.skip_rem) {
+        if (REM && g.skip_rem) {
             const int64_t t = moe_tiled_rows(r.m);
             r.xrows = r.m - t;
             r.m = t;
@@ -1565,8 +1567,13 @@ SRQ_DEV int64_t grouped_tiles(const GroupedProb &r) {
     return ((r.m + kGrpBM - 1) / kGrpBM) * ((r.n + kGrpBN - 1) / kGrpBN);
 }
 
-template <int NPROD, bool UA, int FORM = kFormGeneral, int NSTG = kGrpStages>
-__global__ __launch_bounds__(64 * (4 + NPROD), 1) void gemm_grouped_kernel(GroupedArgs g) {
+// LDS of the grouped kernel: the ring's stages, then the compute waves' int32
+// epilogue blocks (64 x 64 each).
+constexpr int kGrpRing = kGrpStages * kGrpRows * kGrpKBB, kGrpEpi = 4 * (4 * 64 * 64);
+
+// smem: kGrpRing bytes, 1 KiB aligned; epi_lds: kGrpEpi bytes
+template <int NPROD, bool UA, int FORM, int NSTG>
+SRQ_DEV void grouped_body(const GroupedArgs &g, uint8_t *smem, uint8_t *epi_lds) {
     constexpr int WGN = 2, FM = 2, FN = 2, KBB = kGrpKBB;
     static_assert(KBB == 128, "stage layout validated for 128-byte steps only");
     constexpr int kCompute = 4;
@@ -1578,9 +1585,8 @@ __global__ __launch_bounds__(64 * (4 + NPROD), 1) void gemm_grouped_kernel(Group
     static_assert(kDmaPerWave * NPROD == kDma, "DMA split");
     static_assert(NSTG >= 2 && (NSTG - 2) * kDmaPerWave <= 63, "vmcnt range");
     constexpr int kEpiTile = 4 * 32 * FN * 32 * FM;  // a compute wave's int32 block
-    static_assert(NSTG * kStage + kCompute * kEpiTile <= 160 * 1024, "LDS ring");
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[NSTG * kStage];
-    __shared__ __attribute__((aligned(16))) uint8_t epi_lds[kCompute * kEpiTile];
+    static_assert(NSTG * kStage <= kGrpRing && kCompute * kEpiTile <= kGrpEpi &&
+                  kGrpRing + kGrpEpi <= 160 * 1024, "LDS ring");
 
     const int lane0 = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1886,6 +1892,13 @@ __global__ __launch_bounds__(64 * (4 + NPROD), 1) void gemm_grouped_kernel(Group
     }
 }
 
+template <int NPROD, bool UA, int FORM = kFormGeneral, int NSTG = kGrpStages>
+__global__ __launch_bounds__(64 * (4 + NPROD), 1) void gemm_grouped_kernel(GroupedArgs g) {
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[kGrpRing];
+    __shared__ __attribute__((aligned(16))) uint8_t epi_lds[kGrpEpi];
+    grouped_body<NPROD, UA, FORM, NSTG>(g, smem, epi_lds);
+}
+
 // ---------------------------------------------------------------------------
 // Few rows per expert (decode batches), and dense products of 33 to 192 rows
 // (dense_rows, splitk_plan): the grouped kernel's structure with
@@ -1900,22 +1913,25 @@ __global__ __launch_bounds__(64 * (4 + NPROD), 1) void gemm_grouped_kernel(Group
 // own) is hidden and NSTG - 1 steps stay in flight throughout.  An expert
 // with more rows takes several row blocks, adjacent in the tile order so that
 // they read the same weights together.
-// Bound by HBM: gate/up of 8 experts (470 MB) in 100 us, 4.7 TB/s (figures at
+// Bound by HBM: gate/up of 8 experts (470 MB) in 95 us, 4.9 TB/s (figures at
 // moe_row_blocks).
 constexpr int kRowsBN = 128, kRowsKBB = 128;
 
+// LDS of a stage, and of the compute waves' int32 row blocks (32 x 32 each).
+constexpr int rows_stage(int fmb) { return (32 * fmb + kRowsBN) * kRowsKBB; }
+constexpr int kRowsEpi = 4 * (4 * 32 * 32);
+
+// smem: NSTG stages, 1 KiB aligned; epi_lds: kRowsEpi bytes
 template <int FMB, bool UA, int FORM, int NSTG>
-__global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
+SRQ_DEV void rows_body(const GroupedArgs &g, uint8_t *smem, uint8_t *epi_lds) {
     constexpr int BM = 32 * FMB, KBB = kRowsKBB, NPROD = 4, kCompute = 4;
-    constexpr int kStage = (BM + kRowsBN) * KBB;
+    constexpr int kStage = rows_stage(FMB);
     constexpr int C = KBB / 16, R = 1024 / KBB;    // chunks per row, rows per 1 KiB DMA
     constexpr int kAPer = BM / R / NPROD, kBPer = kRowsBN / R / NPROD, kPer = kAPer + kBPer;
     static_assert(kAPer * R * NPROD == BM && kBPer * R * NPROD == kRowsBN, "DMA split");
     static_assert((NSTG - 2) * kPer <= 63, "vmcnt range");
     constexpr int kEpiTile = 4 * 32 * 32;          // a compute wave's int32 row block
-    static_assert(NSTG * kStage + kCompute * kEpiTile <= 160 * 1024, "LDS");
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[NSTG * kStage];
-    __shared__ __attribute__((aligned(16))) uint8_t epi_lds[kCompute * kEpiTile];
+    static_assert(kCompute * kEpiTile == kRowsEpi && NSTG * kStage + kRowsEpi <= 160 * 1024, "LDS");
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1923,7 +1939,7 @@ __global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
     // the experts' concatenated tile lists, row block fastest
     int p = 0;
     int64_t pstart = 0, t = blockIdx.x, m0 = 0, n0 = 0;
-    GroupedProb pr = grouped_prob<FORM>(g, 0);
+    GroupedProb pr = grouped_prob<FORM, false>(g, 0);
     auto tiles_of = [&]() -> int64_t {
         return pr.m <= 0 ? 0 : srq_cdiv(pr.m, BM) * srq_cdiv(pr.n, kRowsBN);
     };
@@ -1932,7 +1948,7 @@ __global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
         while (p < g.P && t >= pstart + ptiles) {
             pstart += ptiles;
             if (++p < g.P) {
-                pr = grouped_prob<FORM>(g, p);
+                pr = grouped_prob<FORM, false>(g, p);
                 ptiles = tiles_of();
             }
         }
@@ -2069,32 +2085,84 @@ __global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
     }
 }
 
-// Launch of FMB = fmb row blocks, ring stages by what LDS holds.
+// Dense and split-K forms (every row of the product in one tile).
+template <int FMB, bool UA, int FORM, int NSTG>
+__global__ __launch_bounds__(512, 1) void gemm_rows_kernel(GroupedArgs g) {
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[NSTG * rows_stage(FMB)];
+    __shared__ __attribute__((aligned(16))) uint8_t epi_lds[kRowsEpi];
+    rows_body<FMB, UA, FORM, NSTG>(g, smem, epi_lds);
+}
+
+// Whether tiles of 32 FMB rows take an expert-offset launch in less time than
+// the 128-row form: by the rounds of the workgroups that the two need, a round
+// of the former at 3/4 (FMB = 1), 7/9, 8/9 or 4/3 (5) of one of the latter.  The
+// rows of each expert are in device memory only, and by their average alone a
+// router that sends most rows to few experts would get many short tiles, each
+// unpacking the weights again.  gate/up / down of 8 experts (4096 / 14336), us, the
+// 128-row form, 32 FMB rows whatever the router, and this rule: 20 rows per expert
+// on average, all on one expert 40 / 70, 63 / 38, 40 / 37, on two (gate/up) 50,
+// 72, 49, as 1 : 1/2 : 1/3 ... (down) 67, 75, 63; 64 on average, on half the
+// experts (gate/up) 98, 130, 98.  1368 launches (six kinds of router, 1 to 200 rows
+// per expert, three expert shapes, four forms) against the 128-row form: 0.87 in
+// the geometric mean, the worst 1.06 where equal kernels differ by up to 1.04; by
+// the average alone the worst was 1.56.
+template <int FMB>
+SRQ_DEV bool rows_win(const GroupedArgs &g) {
+    const int experts = g.pair ? g.P / 2 : g.P;
+    u32 tr = 0, tg = 0;
+    for (int e = threadIdx.x & 63; e < experts; e += 64) {
+        const int m = g.offsets[e + 1] - g.offsets[e];
+        if (m <= 0) continue;
+        const int64_t mg = g.skip_rem ? moe_tiled_rows(m) : m;
+        tr += (u32)(m + 32 * FMB - 1) / (32 * FMB);
+        tg += (u32)(mg + kGrpBM - 1) / kGrpBM;
+    }
+#pragma unroll
+    for (int k = 1; k < 64; k <<= 1) {
+        tr += (u32)__shfl_xor((int)tr, k, 64);
+        tg += (u32)__shfl_xor((int)tg, k, 64);
+    }
+    const uint64_t cols = ((uint64_t)g.N + kRowsBN - 1) / kRowsBN * (g.pair ? 2 : 1);
+    const uint64_t rr = (tr * cols + kGroupedGrid - 1) / kGroupedGrid;
+    const uint64_t rg = (tg * cols + kGroupedGrid - 1) / kGroupedGrid;
+    constexpr int num = FMB == 1 ? 4 : FMB == 2 ? 9 : FMB == 3 ? 9 : 3;
+    constexpr int den = FMB == 1 ? 3 : FMB == 2 ? 7 : FMB == 3 ? 8 : 4;
+    return __builtin_amdgcn_readfirstlane(den * rr <= num * rg);
+}
+
+// Expert-offset forms with few rows per expert on average: the row-block tiles
+// or the 128-row form, by the experts' rows.  One workgroup of either fills the
+// CU's LDS, and which body runs is uniform over the launch.
+template <int FMB, bool UA, int FORM, int NSTG>
+__global__ __launch_bounds__(512, 1) void gemm_moe_kernel(GroupedArgs g) {
+    constexpr int ring = NSTG * rows_stage(FMB);
+    constexpr int bytes = std::max(ring + kRowsEpi, kGrpRing + kGrpEpi);
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[bytes];
+    if (rows_win<FMB>(g)) rows_body<FMB, UA, FORM, NSTG>(g, lds, lds + ring);
+    else grouped_body<4, UA, FORM, kGrpStages>(g, lds, lds + kGrpRing);
+}
+
+// Launch of the dense and split-K forms, all of M in one tile of FMB = fmb row
+// blocks, ring stages by what LDS holds.  Of 97 to 128 rows only the dense
+// SwiGLU form (symmetric activations) comes here.
 template <bool UA, int FORM>
 void launch_rows(const GroupedArgs &g, int fmb, int64_t tiles, hipStream_t st) {
     const dim3 grid((unsigned)std::min<int64_t>(tiles, kGroupedGrid)), block(512);
-    if constexpr (FORM == kFormGeneral || FORM == kFormSwiglu) {
-        if (fmb == 1) gemm_rows_kernel<1, UA, FORM, 7><<<grid, block, 0, st>>>(g);
-        else if (fmb == 2) gemm_rows_kernel<2, UA, FORM, 6><<<grid, block, 0, st>>>(g);
-        else if (FORM == kFormSwiglu || fmb == 3)
-            gemm_rows_kernel<3, UA, FORM, 5><<<grid, block, 0, st>>>(g);
-        else
-            gemm_rows_kernel<5, UA, kFormGeneral, 4><<<grid, block, 0, st>>>(g);
-    } else {
-        if (fmb <= 2) gemm_rows_kernel<2, UA, FORM, 6><<<grid, block, 0, st>>>(g);
-        else if (fmb == 3) gemm_rows_kernel<3, UA, FORM, 5><<<grid, block, 0, st>>>(g);
-        else if (fmb == 4) gemm_rows_kernel<4, UA, FORM, 4><<<grid, block, 0, st>>>(g);
-        else if (fmb == 5) gemm_rows_kernel<5, UA, FORM, 4><<<grid, block, 0, st>>>(g);
-        else gemm_rows_kernel<6, UA, FORM, 3><<<grid, block, 0, st>>>(g);
-    }
+    if (fmb <= 2) gemm_rows_kernel<2, UA, FORM, 6><<<grid, block, 0, st>>>(g);
+    else if (fmb == 3) gemm_rows_kernel<3, UA, FORM, 5><<<grid, block, 0, st>>>(g);
+    else if (fmb == 5) gemm_rows_kernel<5, UA, FORM, 4><<<grid, block, 0, st>>>(g);
+    else if (fmb == 6) gemm_rows_kernel<6, UA, FORM, 3><<<grid, block, 0, st>>>(g);
+    else if constexpr (FORM == kFormDense && !UA)
+        gemm_rows_kernel<4, UA, FORM, 4><<<grid, block, 0, st>>>(g);
 }
 
 // Row blocks (of 32) per tile of an expert-offset launch of `rows` rows over
-// `experts` experts (the rows of each are known on the device only): 1, 2 or
-// 3 on gemm_rows_kernel, 0 for the 128-row kernel.  The lines lie where most
-// experts still fit one row block of a router that is not far from even.
+// `experts` experts (the rows of each are known on the device only): 1, 2, 3 or
+// 5 for gemm_moe_kernel, which takes them if the experts' rows bear it, 0 for
+// the 128-row kernel.  The lines lie where most experts still fit one row block
+// of a router that is not far from even.
 // gate/up + SwiGLU / down of 8 experts (4096 / 14336) against the 128-row
-// kernel, us (one MI355X, two weight sets in turn):
+// kernel, us (one MI355X, two weight sets in turn, random routers):
 //   rows per expert     1           6           24          32          48          64
 //   128-row kernel  105 / 58   141 / 62    138 / 63    138 / 66    145 / 65    150 / 68
 //   1 block          73 / 37   100 / 52    101 / 52    119 / 72    152 / 76    195 / 105
@@ -2107,6 +2175,9 @@ void launch_rows(const GroupedArgs &g, int fmb, int64_t tiles, hipStream_t st) {
 //   rows per expert    120         124         128         136         144         150
 //   128-row kernel  188 / 114   212 / 115   243 / 120   266 / 126   277 / 127   276 / 123
 //   5 blocks        194 / 90    198 / 86    196 / 90    201 / 90    201 / 90    226 / 143
+// (These from gemm_rows_kernel alone.  gemm_moe_kernel with its choice, 1 / 6 / 20 /
+// 48 / 80 rows per expert: gate/up 94 / 95 / 98 / 116 / 143, down 45 / 50 / 50 / 52 / 64,
+// the 128-row kernel then 133 / 135 / 141 / 148 / 154 and 61 / 62 / 65 / 68 / 69.)
 int moe_row_blocks(int64_t rows, int64_t experts, int64_t K, bool extra_rows) {
     if (K < 32) return 0;
     if (!extra_rows && rows > 122 * experts && rows <= 146 * experts) return 5;
@@ -2118,13 +2189,17 @@ int moe_row_blocks(int64_t rows, int64_t experts, int64_t K, bool extra_rows) {
 
 template <bool UA, int FORM>
 void launch_moe(const GroupedArgs &g, int64_t rows, hipStream_t st) {
-    const int fmb = moe_row_blocks(rows, g.pair ? g.P / 2 : g.P, g.K, FORM == kFormSwiglu || g.skip_rem);
-    if (fmb) {
-        GroupedArgs r = g;
-        r.skip_rem = 0;
-        launch_rows<UA, FORM>(r, fmb, kGroupedGrid, st);
-    } else {
-        gemm_grouped_kernel<4, UA, FORM><<<dim3(kGroupedGrid), dim3(512), 0, st>>>(g);
+    const dim3 grid(kGroupedGrid), block(512);
+    switch (moe_row_blocks(rows, g.pair ? g.P / 2 : g.P, g.K,
+                           FORM == kFormSwiglu || g.skip_rem)) {
+    case 1: gemm_moe_kernel<1, UA, FORM, 7><<<grid, block, 0, st>>>(g); break;
+    case 2: gemm_moe_kernel<2, UA, FORM, 6><<<grid, block, 0, st>>>(g); break;
+    case 3: gemm_moe_kernel<3, UA, FORM, 5><<<grid, block, 0, st>>>(g); break;
+    case 5:
+        if constexpr (FORM == kFormGeneral)
+            gemm_moe_kernel<5, UA, FORM, 4><<<grid, block, 0, st>>>(g);
+        break;
+    default: gemm_grouped_kernel<4, UA, FORM><<<grid, block, 0, st>>>(g);
     }
 }
 

@@ -72,3 +72,14 @@ def test_moe_rows_many_experts(C):
         r = slice(bounds[e], bounds[e + 1])
         want = C.w4a4_linear(a[r].contiguous(), sa[r].contiguous(), b[e], sb[e])
         assert torch.equal(out[r], want), f"expert {e}"
+
+
+# routers that send most rows to few experts: by the average these take 32-row to
+# 160-row tiles, by the experts' rows the 128-row form, with and without its extra
+# rows, among empty experts and past 64 of them
+@pytest.mark.parametrize("counts", [[0, 0, 80, 0, 0, 0, 0, 0], [96, 0, 0, 64], [0] * 5 + [129, 0, 0],
+                                    [0, 192, 0, 190], [250, 0, 2, 0], [1, 0, 0, 500],
+                                    [0] * 70 + [640, 3, 0, 130], [128] * 4, [60, 70, 256, 0]])
+@pytest.mark.parametrize("N,K", [(144, 288), (4096, 1024)])
+def test_moe_skewed_bitexact(C, counts, N, K):
+    test_moe_rows_bitexact(C, counts, N, K)
