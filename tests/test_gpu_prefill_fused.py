@@ -216,3 +216,66 @@ def test_prefill_calls_what_is_put_in_place():
     assert torch.equal(out, want) and out.requires_grad
     out.float().sum().backward()
     assert torch.equal(hg.grad, torch.ones_like(hg))   # through the residual adds
+
+
+@pytest.mark.parametrize("dtype", [None, torch.float32])
+def test_fused_prefill_key_rotations(dtype):
+    """Caches whose keys are not rotated, or rotated in fp32."""
+    from signrot_amd.transformers import MultiLayerPagedKVCache4Bit
+    layer, B, T = _layer(1024, 8, 2, 896), 2, 40
+    h = torch.randn(B, T, 1024, device="cuda").half()
+    cos, sin = _cos_sin(B, T, True)
+    outs = []
+    for trace in (None, {}):
+        cache = MultiLayerPagedKVCache4Bit(B, 16, T, "cuda", 1, 2, D, group_size=4,
+                                           hadamard_dtype=dtype)
+        cache.pages.zero_()
+        cache.scales.zero_()
+        outs.append((layer.prefill(h, cache, cos, sin, trace=trace), cache.pages, cache.scales))
+    for a, b in zip(*outs):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+def _wide_layer(hidden, Hq, Hkv, ffn):
+    """Random codes straight on the GPU (random() draws the weights on the CPU)."""
+    from signrot_amd.transformers.decode_layer import W4A4LlamaDecodeLayer
+    layer = W4A4LlamaDecodeLayer(hidden, Hq, Hkv, D, ffn).to("cuda")
+    g = torch.Generator("cuda").manual_seed(7)
+    for name in ("qkv", "o", "gu", "down"):
+        w, s = getattr(layer, f"w_{name}"), getattr(layer, f"s_{name}")
+        w.copy_(torch.randint(0, 256, w.shape, dtype=torch.uint8, device="cuda", generator=g))
+        s.copy_(torch.rand(s.shape, device="cuda", generator=g) * 2e-3 + 1e-3)
+    layer.down_sign.copy_(torch.randint(0, 2, (ffn,), device="cuda", generator=g) * 2 - 1)
+    return layer
+
+
+# 8B widths; an FFN of 172 x 64, whose rotation has no SwiGLU form
+@pytest.mark.parametrize("ffn", [14336, 11008])
+@pytest.mark.parametrize("B,T,padded", [(1, 300, False), (2, 130, True), (1, 2048, False)])
+def test_fused_prefill_model_widths(ffn, B, T, padded):
+    layer = _wide_layer(4096, 32, 8, ffn)
+    h = torch.randn(B, T, 4096, device="cuda", generator=torch.Generator("cuda").manual_seed(T))
+    cos, sin = _cos_sin(B, T, False)
+    mask = None
+    if padded:
+        pad = torch.tensor([[0], [37]], device="cuda")
+        mask = (torch.arange(T, device="cuda")[None] >= pad).int()
+    fused = _run(layer, h.half(), B, T, 256, cos, sin, mask, None)
+    ops = _run(layer, h.half(), B, T, 256, cos, sin, mask, {})
+    for a, b, what in zip(fused, ops, ("hidden", "codes", "params")):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), what
+
+
+def test_prefill_from_two_streams():
+    """One layer, a cache per request, first prefills from two streams at once."""
+    layer, T = _wide_layer(4096, 32, 8, 14336), 512
+    hs = [torch.randn(1, T, 4096, device="cuda").half() for _ in range(2)]
+    cos, sin = _cos_sin(1, T, False)
+    torch.cuda.synchronize()
+    streams, outs = [torch.cuda.Stream() for _ in hs], []
+    for h, s in zip(hs, streams):
+        with torch.cuda.stream(s):
+            outs.append(_prefill(layer, h, cos, sin))
+    torch.cuda.synchronize()
+    for h, out in zip(hs, outs):
+        assert torch.equal(out, _prefill(layer, h, cos, sin))
