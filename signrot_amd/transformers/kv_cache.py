@@ -571,10 +571,13 @@ class MultiLayerPagedKVCache4Bit(Cache):
 def qkv_prefill_of(cache):
     """cache.update_qkv_prefill if it stands for cache.update(), else None: a
     cache without it, or a subclass or an object that has put an update() or
-    a quantizer of its own in place of those that it stands for."""
+    a quantizer of its own in place of those that it stands for, or a key
+    rotation in a type that update() refuses."""
     fill = getattr(cache, "update_qkv_prefill", None)
     base = MultiLayerPagedKVCache4Bit
     if getattr(fill, "__func__", None) is base.update_qkv_prefill:
+        if cache.hadamard_dtype not in (None, torch.float16, torch.float32):
+            return None
         for name in ("update", "_quantize"):
             if getattr(getattr(cache, name), "__func__", None) is not getattr(base, name):
                 return None

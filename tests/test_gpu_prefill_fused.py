@@ -279,3 +279,17 @@ def test_prefill_from_two_streams():
     torch.cuda.synchronize()
     for h, out in zip(hs, outs):
         assert torch.equal(out, _prefill(layer, h, cos, sin))
+
+
+def test_prefill_refuses_other_key_rotations():
+    """A key rotation in a type that the Hadamard kernel has not is refused by
+    a prefill, and nothing comes into the cache."""
+    from signrot_amd.transformers import MultiLayerPagedKVCache4Bit
+    layer, T = _layer(1024, 8, 2, 896), 8
+    cos, sin = _cos_sin(1, T, False)
+    h = torch.randn(1, T, 1024, device="cuda").half()
+    cache = MultiLayerPagedKVCache4Bit(1, 16, T, "cuda", 1, 2, D, group_size=4,
+                                       hadamard_dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError, match="only float16 and float32"):
+        layer.prefill(h, cache, cos, sin)
+    assert cache.length == 0 and not any(cache._filled)
