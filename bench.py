@@ -601,23 +601,31 @@ def traffic_commit():
 
 def gemm_kernel_name(M, N, K=None, split=False):
     """Kernel srq_w4a4_linear(_ws) launches for M x N outputs (gemm.hip
-    dispatch, fp16 output)."""
+    dispatch, fp16 output; split: the shape has a workspace)."""
     def cdiv(a, b):
         return -(-a // b)
     if M <= 32:
         return "gemm_stream_kernel (srq_w4a4_linear)"
-    if 32 < M <= 96 and split:
-        return "gemm_rows_kernel split-K form + splitk_reduce_kernel (srq_w4a4_linear_ws)"
+    ct = cdiv(N, 128)
+    if (M <= 96 or 128 < M <= 192) and ct >= 192:
+        return "gemm_rows_kernel (srq_w4a4_linear)"
+    if split:
+        few = M <= 96 and (M > 64 or cdiv(cdiv(N, 16), 256) * K > 8192)
+        wide = 128 < M <= (160 if ct >= 96 else 192)
+        chunks = min(256 // ct, K // (1280 if few else 4096)) if few or wide else 0
+        if chunks >= 2 and ct * chunks >= (200 if wide and ct <= 64 else 160):
+            return "gemm_rows_kernel split-K form + splitk_reduce_kernel (srq_w4a4_linear_ws)"
     if M <= 64:
         return "gemm_skinny_kernel (srq_w4a4_linear)"
-    sq, big = cdiv(M, 256) * cdiv(N, 256), cdiv(M, 256) * cdiv(N, 128)
+    tiles, sq, big = cdiv(M, 128) * ct, cdiv(M, 256) * cdiv(N, 256), cdiv(M, 256) * ct
     if M >= 1024 and 7 * cdiv(sq, 256) <= 4 * cdiv(big, 256):
         return "gemm_sq_kernel (srq_w4a4_linear, 256 x 256 tiles)"
     if split:
-        return "gemm_grouped_kernel split-K form + splitk_reduce_kernel (srq_w4a4_linear_ws)"
-    if M < 1024 and cdiv(M, 128) * cdiv(N, 128) >= 192 and cdiv(M, 256) * cdiv(N, 128) < 512:
+        kernel = "gemm_big_kernel" if tiles >= 192 else "gemm_grouped_kernel"
+        return f"{kernel} split-K form + splitk_reduce_kernel (srq_w4a4_linear_ws)"
+    if M < 1024 and tiles >= 192 and big < 512:
         return "gemm_grouped_kernel dense form (srq_w4a4_linear, 128 x 128 tiles)"
-    if M >= 1024 or cdiv(M, 256) * cdiv(N, 128) >= 512:
+    if M >= 1024 or big >= 512:
         return "gemm_big_kernel (srq_w4a4_linear, 256 x 128 tiles)"
     return "gemm_ring_kernel (srq_w4a4_linear)"
 
