@@ -1473,7 +1473,6 @@ struct GroupedArgs {
     // residual [M, N] (either may be null)
     int64_t M;
     const f16 *bias, *res;
-    int swiglu;  // dense form: the columns are blocks of 8 gate, 8 up; out [M, N/2]
     int64_t ldo;  // dense swiglu form: Epi::ldo
     // split-K form (the SPLITK instantiation): problem p is the dense
     // product over K codes [p Kc, min((p + 1) Kc, K)), its int32 partial
@@ -1483,8 +1482,11 @@ struct GroupedArgs {
 };
 
 // kFormSwiglu: the expert-offset form over gate/up rows interleaved in
-// blocks of 8, out [R, N/2] = swiglu(gate, up)
-constexpr int kFormGeneral = 0, kFormDense = 1, kFormSplitK = 2, kFormSwiglu = 3;
+// blocks of 8, out [R, N/2] = swiglu(gate, up); kFormDenseSwiglu: the dense one
+constexpr int kFormGeneral = 0, kFormDense = 1, kFormSplitK = 2, kFormSwiglu = 3,
+              kFormDenseSwiglu = 4;
+constexpr bool form_dense(int form) { return form == kFormDense || form == kFormDenseSwiglu; }
+constexpr bool form_swiglu(int form) { return form == kFormSwiglu || form == kFormDenseSwiglu; }
 
 struct GroupedProb {
     const uint8_t *a, *b;
@@ -1519,7 +1521,7 @@ SRQ_DEV GroupedProb grouped_prob(const GroupedArgs &g, int p) {
         r.ldc = g.N;
         return r;
     }
-    if constexpr (FORM == kFormDense) {
+    if constexpr (form_dense(FORM)) {
         r.row0 = 0;
         r.m = g.M;
         r.n = g.N;
@@ -1846,16 +1848,16 @@ SRQ_DEV void grouped_body(const GroupedArgs &g, uint8_t *smem, uint8_t *epi_lds)
             // through the wave's own LDS tile (the ring's stages already
             // take the next tile's DMA); the sym_dequant_moe zero correction
             // is epi_val's
-            constexpr bool DENSE = FORM == kFormDense;
+            constexpr bool DENSE = form_dense(FORM);
             const bool second = !DENSE && g.pair && (p & 1);
             const int64_t ex = DENSE ? 0 : g.pair ? p >> 1 : p;
             Epi e{};
-            const bool sw = FORM == kFormSwiglu || (DENSE && g.swiglu);
+            constexpr bool sw = form_swiglu(FORM);
             e.out = (second ? g.out2 : g.out) + pr.row0 * (sw ? g.N / 2 : g.N);
             e.sa = g.sa + pr.row0;
             e.sb = (second ? g.sb2 : g.sb) + ex * g.N;
             e.ua = UA;
-            if (g.zr) {
+            if (UA && g.zr) {
                 e.zr = g.zr + pr.row0;
                 e.ws = (second ? g.ws2 : g.ws) + ex * g.N;
             }
@@ -1864,7 +1866,7 @@ SRQ_DEV void grouped_body(const GroupedArgs &g, uint8_t *smem, uint8_t *epi_lds)
                 e.res = g.res;
                 e.ldo = g.ldo;
             }
-            if (sw)
+            if constexpr (sw)
                 store_block_lds32_swiglu<32, FM, FN>(
                     e, pr.m, pr.n, m0 + wm * (FM * 32), n0 + wn * (FN * 32), acc, lane,
                     reinterpret_cast<int32_t *>(epi_lds + wave * kEpiTile));
@@ -2051,16 +2053,16 @@ SRQ_DEV void rows_body(const GroupedArgs &g, uint8_t *smem, uint8_t *epi_lds) {
             }
             continue;
         }
-        constexpr bool DENSE = FORM == kFormDense;
+        constexpr bool DENSE = form_dense(FORM);
         const bool second = !DENSE && g.pair && (p & 1);
         const int64_t ex = DENSE ? 0 : g.pair ? p >> 1 : p;
-        const bool sw = FORM == kFormSwiglu || (DENSE && g.swiglu);
+        constexpr bool sw = form_swiglu(FORM);
         Epi e{};
         e.out = (second ? g.out2 : g.out) + pr.row0 * (sw ? g.N / 2 : g.N);
         e.sa = g.sa + pr.row0;
         e.sb = (second ? g.sb2 : g.sb) + ex * g.N;
         e.ua = UA;
-        if (g.zr) {
+        if (UA && g.zr) {
             e.zr = g.zr + pr.row0;
             e.ws = (second ? g.ws2 : g.ws) + ex * g.N;
         }
@@ -2075,7 +2077,7 @@ SRQ_DEV void rows_body(const GroupedArgs &g, uint8_t *smem, uint8_t *epi_lds) {
         for (int i = 0; i < FMB; ++i) {
             const v16i one[1][1] = {{acc[i][0]}};
             if (m0 + 32 * i >= pr.m) break;
-            if (sw)
+            if constexpr (sw)
                 store_block_lds32_swiglu<32, 1, 1>(e, pr.m, pr.n, m0 + 32 * i, n0 + wave * 32, one,
                                                    lane, tile);
             else
@@ -2152,7 +2154,7 @@ void launch_rows(const GroupedArgs &g, int fmb, int64_t tiles, hipStream_t st) {
     else if (fmb == 3) gemm_rows_kernel<3, UA, FORM, 5><<<grid, block, 0, st>>>(g);
     else if (fmb == 5) gemm_rows_kernel<5, UA, FORM, 4><<<grid, block, 0, st>>>(g);
     else if (fmb == 6) gemm_rows_kernel<6, UA, FORM, 3><<<grid, block, 0, st>>>(g);
-    else if constexpr (FORM == kFormDense && !UA)
+    else if constexpr (FORM == kFormDenseSwiglu)
         gemm_rows_kernel<4, UA, FORM, 4><<<grid, block, 0, st>>>(g);
 }
 
@@ -2452,7 +2454,6 @@ GroupedArgs dense_args(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N,
     g.res = e.res;
     g.zr = e.zr;
     g.ws = e.ws;
-    g.swiglu = e.swiglu;
     g.ldo = e.ldo;
     return g;
 }
@@ -2471,7 +2472,15 @@ void launch_gemm(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64
         // M <= 32: persistent weight-streaming kernel
     } else if (!e.C && dense_rows(M, N, K, e.swiglu != 0)) {
         GroupedArgs g = dense_args(a, b, M, N, K, e);
-        launch_rows<UA, kFormDense>(g, (int)srq_cdiv(M, 32), srq_cdiv(N, kRowsBN), st);
+        const int fmb = (int)srq_cdiv(M, 32);
+        const int64_t tiles = srq_cdiv(N, kRowsBN);
+        if constexpr (!UA) {
+            if (e.swiglu) {
+                launch_rows<UA, kFormDenseSwiglu>(g, fmb, tiles, st);
+                return;
+            }
+        }
+        launch_rows<UA, kFormDense>(g, fmb, tiles, st);
     } else if (sk.S && sk.rows && !e.swiglu && ws_bytes >= (int64_t)sk.S * M * N * 4) {
         GroupedArgs g = dense_args(a, b, M, N, K, Epi{});
         g.P = sk.S;
@@ -2521,8 +2530,17 @@ void launch_gemm(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64
         // nibble unpacking: 188 -> 113 us at M = 512, N = 8192, K = 28672)
         const GroupedArgs g = dense_args(a, b, M, N, K, e);
         const int64_t tiles = srq_cdiv(M, kGrpBM) * srq_cdiv(N, kGrpBN);
-        gemm_grouped_kernel<4, UA, kFormDense>
-            <<<dim3((unsigned)std::min<int64_t>(tiles, kGroupedGrid)), dim3(512), 0, st>>>(g);
+        const dim3 grid((unsigned)std::min<int64_t>(tiles, kGroupedGrid)), block(512);
+        // The SwiGLU form apart: with both epilogues in one kernel the compute
+        // waves' loop constants spill (78 SGPRs, 24 here): N = 57344, K = 8192, M = 201
+        // 150 -> 143 us, N = 28672, K = 4096, M = 512 85.5 -> 80.
+        if constexpr (!UA) {
+            if (e.swiglu) {
+                gemm_grouped_kernel<4, UA, kFormDenseSwiglu><<<grid, block, 0, st>>>(g);
+                return;
+            }
+        }
+        gemm_grouped_kernel<4, UA, kFormDense><<<grid, block, 0, st>>>(g);
     } else if (M >= 1024 || srq_cdiv(M, kBigBM) * srq_cdiv(N, kBigBN) >= 512) {
         const int64_t tm = srq_cdiv(M, kBigBM), tiles = tm * srq_cdiv(N, kBigBN);
         const int64_t rem = tiles % 256;
