@@ -33,6 +33,7 @@ import torch
 from .. import _CUDA
 from ..functional import kernel
 from ..functional.hadamard import get_hadK, matmul_hadU_cuda
+from .derived import derived
 
 
 class MoERouting(NamedTuple):
@@ -260,12 +261,8 @@ class SignRotMoEBlock(torch.nn.Module):
         the blocks-of-8 layout of w4a4_linear_moe_swiglu: a derived copy,
         made on first use and again whenever a source buffer changes in
         place."""
-        src = (self.w_gate, self.s_gate, self.w_up, self.s_up)
-        key = tuple((t.data_ptr(), t._version) for t in src)
-        if getattr(self, "_gu_il_key", None) != key:
-            self._gu_il = _CUDA.interleave_gate_up_experts(*src)
-            self._gu_il_key = key
-        return self._gu_il
+        return derived(self, "_gu_il", (self.w_gate, self.s_gate, self.w_up, self.s_up),
+                       _CUDA.interleave_gate_up_experts)
 
     def _combine(self, x, shape, y, route: MoERouting):
         """Expert-ordered rows y back to tokens, weighted and summed over

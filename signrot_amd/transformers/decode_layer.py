@@ -22,6 +22,7 @@ from .. import _CUDA
 from ..functional import kernel
 from ..functional.hadamard import _inv_sqrt_f32, get_hadK, matmul_hadU_cuda
 from ..functional.quantization import rtn_weight_pack
+from ..nn.derived import derived
 from ..nn.normalization import RMSNorm
 from .kv_cache import qkv_prefill_of
 
@@ -87,12 +88,8 @@ class W4A4LlamaDecodeLayer(torch.nn.Module):
         """w_gu / s_gu in the blocks-of-8 gate/up layout of
         w4a4_linear_swiglu: a derived copy (2 ffn x hidden / 2 bytes), made
         on first use and again whenever w_gu or s_gu changes in place."""
-        key = (self.w_gu.data_ptr(), self.w_gu._version, self.s_gu.data_ptr(),
-               self.s_gu._version)
-        if getattr(self, "_gu_il_key", None) != key:
-            self._gu_il = _CUDA.interleave_gate_up(self.w_gu, self.s_gu, self.ffn)
-            self._gu_il_key = key
-        return self._gu_il
+        return derived(self, "_gu_il", (self.w_gu, self.s_gu),
+                       lambda w, s: _CUDA.interleave_gate_up(w, s, self.ffn))
 
     def _linear(self, xq, name):
         q, s = xq.quantized_x, xq.scales_x
