@@ -2152,10 +2152,16 @@ void launch_rows(const GroupedArgs &g, int fmb, int64_t tiles, hipStream_t st) {
     const dim3 grid((unsigned)std::min<int64_t>(tiles, kGroupedGrid)), block(512);
     if (fmb <= 2) gemm_rows_kernel<2, UA, FORM, 6><<<grid, block, 0, st>>>(g);
     else if (fmb == 3) gemm_rows_kernel<3, UA, FORM, 5><<<grid, block, 0, st>>>(g);
-    else if (fmb == 5) gemm_rows_kernel<5, UA, FORM, 4><<<grid, block, 0, st>>>(g);
     else if (fmb == 6) gemm_rows_kernel<6, UA, FORM, 3><<<grid, block, 0, st>>>(g);
-    else if constexpr (FORM == kFormDenseSwiglu)
-        gemm_rows_kernel<4, UA, FORM, 4><<<grid, block, 0, st>>>(g);
+    else {
+        if constexpr (FORM == kFormDenseSwiglu) {
+            if (fmb == 4) {
+                gemm_rows_kernel<4, UA, FORM, 4><<<grid, block, 0, st>>>(g);
+                return;
+            }
+        }
+        gemm_rows_kernel<5, UA, FORM, 4><<<grid, block, 0, st>>>(g);
+    }
 }
 
 // Row blocks (of 32) per tile of an expert-offset launch of `rows` rows over
@@ -2197,10 +2203,12 @@ void launch_moe(const GroupedArgs &g, int64_t rows, hipStream_t st) {
     case 1: gemm_moe_kernel<1, UA, FORM, 7><<<grid, block, 0, st>>>(g); break;
     case 2: gemm_moe_kernel<2, UA, FORM, 6><<<grid, block, 0, st>>>(g); break;
     case 3: gemm_moe_kernel<3, UA, FORM, 5><<<grid, block, 0, st>>>(g); break;
-    case 5:
-        if constexpr (FORM == kFormGeneral)
+    case 5:   // of the general form only
+        if constexpr (FORM == kFormGeneral) {
             gemm_moe_kernel<5, UA, FORM, 4><<<grid, block, 0, st>>>(g);
-        break;
+            break;
+        }
+        [[fallthrough]];
     default: gemm_grouped_kernel<4, UA, FORM><<<grid, block, 0, st>>>(g);
     }
 }
