@@ -618,7 +618,8 @@ def gemm_kernel_name(M, N, K=None, split=False):
     if M <= 64:
         return "gemm_skinny_kernel (srq_w4a4_linear)"
     tiles, sq, big = cdiv(M, 128) * ct, cdiv(M, 256) * cdiv(N, 256), cdiv(M, 256) * ct
-    if M >= 1024 and 7 * cdiv(sq, 256) <= 4 * cdiv(big, 256):
+    num, den = (7, 4) if K is None or K >= 4096 else (5, 3) if K >= 2048 else (3, 2)
+    if M >= 1024 and num * cdiv(sq, 256) <= den * cdiv(big, 256):
         return "gemm_sq_kernel (srq_w4a4_linear, 256 x 256 tiles)"
     if split:
         kernel = "gemm_big_kernel" if tiles >= 192 else "gemm_grouped_kernel"

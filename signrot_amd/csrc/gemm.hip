@@ -2434,15 +2434,20 @@ void splitk_reduce(const void *ws, int S, int64_t M, int64_t N, const Epi &e, hi
 
 // Square or 256 x 128 tiles for a large product: by the rounds of the 256 CUs
 // that each takes, a round of square tiles being about 1.75 of the others
-// (twice the work, less data movement); square where they tie.  us, K = 4096,
-// weights from memory: M = 2048, N = 6144 (192 against 384 tiles) square 53,
+// (twice the work, less data movement), 5/3 below K = 4096 and 1.5 below 2048,
+// where the epilogue's share of a round grows; square where they tie.  us, K =
+// 4096, weights from memory: M = 2048, N = 6144 (192 against 384 tiles) square 53,
 // 256 x 128 58; M = 1500, N = 6144 55, 61; M = 1024, N = 14336 (224, 448) 57, 63;
 // M = 1200, N = 28672 (560, 1120) 163, 159; M = 2048, N = 28672 (896, 1792; tie)
-// 228, 241; M = 2048, N = 4096 (128, 256) 51, 35.
-bool use_square_tiles(int64_t M, int64_t N) {
+// 228, 241; M = 2048, N = 4096 (128, 256) 51, 35.  256 x 128 tiles over square ones,
+// mean and worst of 24 to 74 shapes: 2 against 3 rounds, K = 1024 / 2048 / 4096 1.01,
+// 0.94, 0.88 (1.13, 1.02, 0.96); 3 against 5, K = 2048 / 3072 / 4096 1.01, 0.98,
+// 0.96 (1.05, 1.03, 1.00).
+bool use_square_tiles(int64_t M, int64_t N, int64_t K) {
     const int64_t sq = srq_cdiv(M, kSqBM) * srq_cdiv(N, kSqBN);
     const int64_t big = srq_cdiv(M, kBigBM) * srq_cdiv(N, kBigBN);
-    return 7 * srq_cdiv(sq, 256) <= 4 * srq_cdiv(big, 256);
+    const int num = K < 2048 ? 3 : K < 4096 ? 5 : 7, den = K < 2048 ? 2 : K < 4096 ? 3 : 4;
+    return num * srq_cdiv(sq, 256) <= den * srq_cdiv(big, 256);
 }
 
 // One dense problem with e's fp16 epilogue.
@@ -2505,7 +2510,7 @@ void launch_gemm(const uint8_t *a, const uint8_t *b, int64_t M, int64_t N, int64
     } else if (M <= 64 && !e.swiglu) {
         gemm_skinny_kernel<4, 8, 2, UA><<<dim3((unsigned)srq_cdiv(N, 16), 1), dim3(512), 0, st>>>(
             a, b, M, N, K, e);
-    } else if (M >= 1024 && use_square_tiles(M, N)) {
+    } else if (M >= 1024 && use_square_tiles(M, N, K)) {
         const int64_t tiles = srq_cdiv(M, kSqBM) * srq_cdiv(N, kSqBN);
         gemm_sq_kernel<128, 2, UA><<<dim3((unsigned)tiles), dim3(512), 0, st>>>(a, b, M, N, K, e);
     } else if (sk.S && sk.big && !e.swiglu && ws_bytes >= (int64_t)sk.S * M * N * 4) {
